@@ -2,41 +2,35 @@
 // (src/dsine_refine.cpp:161-294) on one HIP device, over this library's C ABI
 // (include/bvml_dsine.h).
 //
-// Once per forward, the ConvGRU convolutions' parts over [feature | uv], the
-// channels no iteration changes (conv(cat(h, x), W) = conv(h, W_h) + conv(x,
-// W_x)):
-//   cf_zr = conv5x5([feature | uv], [W_z; W_r] over those channels), cf_q likewise
-//                                                            bvml_dsine_conv_f32
-// Per iteration (src/dsine_refine.cpp:255-287), on persistent per-grid maps:
-//   z, r*h = gates of conv5x5(h, [W_z; W_r] over h) + cf_zr  bvml_dsine_conv_gru_gates_sum_f32
-//   h    = (1 - z) h + z tanh(conv5x5(r*h, W_q over h) + cf_q + b_q),
-//          also into [h | uv]                                bvml_dsine_conv_gru_update_sum_f32
+// Once per forward:
+//   the ray and uv maps, pred = RayReLU(normal, ray)  (src/dsine_refine.cpp:240-242),
+//   the hidden state and the features as split maps (refiner_conv.hip)
+//   cf = conv5x5([feature | uv], [W_z; W_r; W_q] over those channels): the
+//        ConvGRU convolutions' parts over the channels no iteration changes
+//        (conv(cat(h, x), W) = conv(h, W_h) + conv(x, W_x))
+// Per iteration (:255-287), on persistent per-grid maps:
+//   z, r*h = gates of conv5x5(h, [W_z; W_r] over h) + cf
+//   h    = (1 - z) h + z tanh(conv5x5(r*h, W_q over h) + cf + b_q)
 //   prob, xy, angle = the three heads (conv3x3 -> ReLU -> conv1x1 -> ReLU -> conv1x1)
-//          on [h | uv], the 1x1 layers in the 3x3 layer's epilogue
-//                                                            bvml_dsine_conv_heads_f32, 66 -> 192
-//          (last iteration, all four heads: t0 = conv3x3, 66 -> 256, then the 1x1 layers
-//          on relu(t0 + b0)                     bvml_dsine_conv_f32, bvml_dsine_heads_mlp_f32)
+//          on [h | uv], the 1x1 layers in the 3x3 layer's epilogue (the last
+//          iteration: all four heads)
 //   pred = angmf_propagate(pred, prob, xy, angle) on logits  bvml_dsine_angmf_propagate_f32
-// and, in the last iteration only, the up-mask head (its 1x1 layers in the
-// same heads pass) and the convex upsample + normalise with its bias (the
-// reference computes
-// an up-sampled map every iteration but returns the last one only,
-// src/dsine_refine.cpp:276-283, :289-293, so the others are dead work).  In
-// the first four iterations the heads run for the three heads the propagate
-// reads (their 3x3 layer at 192 channels); the last iteration runs all four
-// (256).  The convolutions run without their bias; the fused kernels add it
-// in the reference's rounding (a bias add after the convolution's sum).
+// and, in the last iteration only, the up-mask head and the convex upsample +
+// normalise with its bias (the reference computes an up-sampled map every
+// iteration but returns the last one only, :276-283, :289-293, so the others
+// are dead work).  The convolutions add their bias once after their sum, in
+// the reference's rounding.
 //
-// Every convolution is this library's implicit GEMM on the fp32 matrix cores
-// (conv.hip): the kernels, their launch shapes and so their summation order
-// depend on the grid size only, so a forward's result is the same in every
-// process and from both forward entry points (a library that picks its
-// algorithm by measured or estimated time, as MIOpen's immediate mode does,
-// changes its rounding with the process's history).  The maps are allocated
-// once per grid size.
+// Every convolution is the library's own implicit GEMM: the kernels, their
+// launch shapes and so their summation order depend on the grid size only, so
+// a forward's result is the same in every process and from both forward entry
+// points (a library that picks its algorithm by measured or estimated time, as
+// MIOpen's immediate mode does, changes its rounding with the process's
+// history).  The maps are allocated once per grid size.
 
 #include "bvml_dsine_refine.h"
 #include "refiner_common.h"
+#include "refiner_kernels.h"
 
 #include <hip/hip_runtime.h>
 
@@ -61,6 +55,11 @@ int fail(int code, const std::string& msg) {
 }
 
 const char* last_error() { return g_last_error.c_str(); }
+
+const Kernels*& kernels() {
+    static const Kernels* k = nullptr;
+    return k;
+}
 
 bool overlaps(const void* a, size_t abytes, const void* b, size_t bbytes) {
     const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
@@ -138,6 +137,7 @@ int check_forward(const std::vector<std::vector<float>>& host, const ForwardArgs
 namespace {
 
 using namespace bvml_refine;
+static_assert(kInfoFloats == kInfoWords, "room for the scales");
 
 // ---------------------------------------------------------------------------
 // safetensors: an 8-byte little-endian header length, a JSON header mapping
@@ -515,18 +515,15 @@ struct bvml_dsine_refiner {
 
     // weights on the device, one allocation
     float* warena = nullptr;
-    // convz + convr and convq, each split by input channels into the part
-    // over h (every iteration) and the part over [feature | uv] (once per
-    // forward), packed for the implicit-GEMM kernels
-    const float *w_zr_h = nullptr, *w_zr_f = nullptr, *b_z = nullptr, *b_r = nullptr;
-    const float *w_q_h = nullptr, *w_q_f = nullptr, *b_q = nullptr;
-    const float *b_h0 = nullptr, *w2p = nullptr, *b_h2 = nullptr;
-    // the three propagate heads' middle layers in the last-layer layout, for
-    // bvml_dsine_conv_heads_f32
-    const float* w2q = nullptr;
-    const float* w_h0p[2] = {};  // the 3x3 layer packed for bvml_dsine_conv_f32 (192, 256 filters)
-    const float* w4p[kHeads] = {};  // the 1x1 layers packed for bvml_dsine_heads_mlp_f32
-    const float* b4[kHeads] = {};
+    // packed for refiner_conv.hip: the ConvGRU's filters over [feature | uv]
+    // (convz and convr in alternating blocks of 16, then convq), over h (convz
+    // and convr alike), over r*h (convq); the heads' 3x3 layers; their 1x1
+    // layers
+    const float *w_ctx = nullptr, *w_zr = nullptr, *w_q = nullptr, *w_h0 = nullptr;
+    const float *b_z = nullptr, *b_r = nullptr, *b_q = nullptr;
+    const float* w2[kHeads] = {};
+    const float* w4[kHeads] = {};
+    const float* b_h[kHeads][3] = {};
 
     // the maps of one grid size, one allocation
     int H = 0, W = 0;
@@ -546,128 +543,45 @@ struct bvml_dsine_refiner {
         if (warena) (void)hipFree(warena);
     }
 
-    int upload();
+    int upload(hipStream_t stream);
     int plan(int H, int W);
 };
 
-// Copies the host weights into the device arena, in the layout the kernels
-// read: [W_z; W_r] as one 128-filter weight, the four heads' first layers as
-// one 192- and one 256-filter weight (each head's filters contiguous, prob,
-// xy, angle, up_mask: the first three heads are a prefix), all three packed
-// for bvml_dsine_conv_*, and the heads' 1x1 layers packed for
-// bvml_dsine_heads_mlp_f32 (and the first three heads' middle layers again,
-// in the last-layer layout, for bvml_dsine_conv_heads_f32).
-int bvml_dsine_refiner::upload() {
-    std::vector<float> w2(kHeads * kMid * kMid), w2p_h((size_t)kHeads * 4096);
-    std::vector<std::vector<float>> w4p_h(kHeads);
-    const float* w4src[kHeads];
-    float* w4dst[kHeads];
-    for (int h = 0; h < kHeads; ++h) {
-        std::memcpy(&w2[(size_t)h * kMid * kMid], host[head_w(h, 1)].data(),
-                    (size_t)kMid * kMid * sizeof(float));
-        w4p_h[h].resize((size_t)bvml_dsine_heads_packed_size(kHeadOut[h]));
-        w4src[h] = host[head_w(h, 2)].data();
-        w4dst[h] = w4p_h[h].data();
-    }
-    if (const int st = bvml_dsine_heads_pack_f32(w2.data(), w4src, kHeadOut, kHeads, w2p_h.data(),
-                                                 w4dst))
-        return fail(st, std::string("forward: heads_pack: ") + bvml_dsine_last_error());
-    // W2 of each of the first three heads packed as a 64-output last layer
-    constexpr int kProp = kHeads - 1;
-    const long long w2q_n = bvml_dsine_heads_packed_size(kMid);
-    std::vector<float> w2q_h((size_t)kProp * w2q_n), w2p_tmp((size_t)kProp * 4096);
-    {
-        const float* src[kProp];
-        float* dst[kProp];
-        int outs[kProp];
-        for (int h = 0; h < kProp; ++h) {
-            src[h] = &w2[(size_t)h * kMid * kMid];
-            dst[h] = &w2q_h[(size_t)h * w2q_n];
-            outs[h] = kMid;
-        }
-        if (const int st = bvml_dsine_heads_pack_f32(w2.data(), src, outs, kProp, w2p_tmp.data(),
-                                                     dst))
-            return fail(st, std::string("forward: heads_pack: ") + bvml_dsine_last_error());
-    }
-    // [W_z; W_r] with their 16-channel blocks interleaved, and W_q, each as
-    // its input channels [0, kHidden) (h) and [kHidden, kHx) (feature, uv):
-    // conv(cat(h, x), W) = conv(h, W_h) + conv(x, W_x)
-    std::vector<float> wzr(host[kZw]);
-    wzr.insert(wzr.end(), host[kRw].begin(), host[kRw].end());
-    auto in_slice = [](const std::vector<float>& w, int cout, int c0, int c1) {
-        std::vector<float> out;
-        out.reserve((size_t)cout * (c1 - c0) * 25);
-        for (int o = 0; o < cout; ++o)
-            out.insert(out.end(), w.begin() + ((size_t)o * kHx + c0) * 25,
-                       w.begin() + ((size_t)o * kHx + c1) * 25);
-        return out;
-    };
-    std::vector<float> wsplit_p[4];
-    {
-        const std::vector<float>* src[4] = {&wzr, &wzr, &host[kQw], &host[kQw]};
-        const int cout[4] = {2 * kHidden, 2 * kHidden, kHidden, kHidden};
-        const int c0[4] = {0, kHidden, 0, kHidden}, c1[4] = {kHidden, kHx, kHidden, kHx};
-        const int il[4] = {1, 1, 0, 0};
-        for (int i = 0; i < 4; ++i) {
-            const std::vector<float> w = in_slice(*src[i], cout[i], c0[i], c1[i]);
-            wsplit_p[i].resize((size_t)bvml_dsine_conv_packed_size(cout[i], c1[i] - c0[i], 5));
-            if (const int st = bvml_dsine_conv_pack_f32(w.data(), cout[i], c1[i] - c0[i], 5, il[i],
-                                                        wsplit_p[i].data()))
-                return fail(st, std::string("forward: conv_pack: ") + bvml_dsine_last_error());
-        }
-    }
-    std::vector<float> wh0;
-    for (int h = 0; h < kHeads; ++h)
-        wh0.insert(wh0.end(), host[head_w(h, 0)].begin(), host[head_w(h, 0)].end());
-    std::vector<float> wh0_p[2];
-    for (int i = 0; i < 2; ++i) {
-        const int co = (3 + i) * kMid;
-        wh0_p[i].resize((size_t)bvml_dsine_conv_packed_size(co, kHin, 3));
-        if (const int st = bvml_dsine_conv_pack_f32(wh0.data(), co, kHin, 3, 0, wh0_p[i].data()))
-            return fail(st, std::string("forward: conv_pack: ") + bvml_dsine_last_error());
-    }
-    using Src = std::vector<const std::vector<float>*>;
-    std::vector<std::pair<const float**, Src>> parts;
-    parts.push_back({&w_zr_h, {&wsplit_p[0]}});
-    parts.push_back({&w_zr_f, {&wsplit_p[1]}});
-    parts.push_back({&b_z, {&host[kZb]}});
-    parts.push_back({&b_r, {&host[kRb]}});
-    parts.push_back({&w_q_h, {&wsplit_p[2]}});
-    parts.push_back({&w_q_f, {&wsplit_p[3]}});
-    parts.push_back({&b_q, {&host[kQb]}});
-    Src h0b, h2b;
-    for (int h = 0; h < kHeads; ++h) {
-        h0b.push_back(&host[head_b(h, 0)]);
-        h2b.push_back(&host[head_b(h, 1)]);
-    }
-    parts.push_back({&w_h0p[0], {&wh0_p[0]}});
-    parts.push_back({&w_h0p[1], {&wh0_p[1]}});
-    parts.push_back({&b_h0, h0b});
-    parts.push_back({&w2p, {&w2p_h}});
-    parts.push_back({&w2q, {&w2q_h}});
-    parts.push_back({&b_h2, h2b});
-    for (int h = 0; h < kHeads; ++h) {
-        parts.push_back({&w4p[h], {&w4p_h[h]}});
-        parts.push_back({&b4[h], {&host[head_b(h, 2)]}});
-    }
-    std::vector<size_t> offset;
+// Copies the host weights to the device and packs them there
+// (refiner_kernels.h): the ConvGRU's filters over their input channels
+// [0, kHidden) (h) and [kHidden, kHx) (feature, uv) apart, since conv(cat(h, x),
+// W) = conv(h, W_h) + conv(x, W_x).
+int bvml_dsine_refiner::upload(hipStream_t stream) {
+    const Kernels* kern = kernels();
+    if (!kern) return fail(BVML_DSINE_EUNSUP, "forward: built without the device kernels");
+    const size_t ns = specs().size();
+    std::vector<size_t> at(ns);
     size_t total = 0;
-    for (const auto& p : parts) {
-        offset.push_back(total);
-        size_t n = 0;
-        for (const std::vector<float>* v : p.second) n += v->size();
-        total += round64(n);
+    for (size_t i = 0; i < ns; ++i) {
+        at[i] = total;
+        total += round64(host[i].size());
     }
-    std::vector<float> staging(total, 0.0f);
-    for (size_t k = 0; k < parts.size(); ++k) {
-        size_t at = offset[k];
-        for (const std::vector<float>* v : parts[k].second) {
-            std::memcpy(&staging[at], v->data(), v->size() * sizeof(float));
-            at += v->size();
-        }
+    const size_t raw = total;
+    auto room = [&](size_t words) {
+        const size_t place = total;
+        total += round64(words);
+        return place;
+    };
+    const size_t p_ctx = room(split_words(3 * kHidden, 5, true));
+    const size_t p_zr = room(split_words(2 * kHidden, 5, false));
+    const size_t p_q = room(split_words(kHidden, 5, false));
+    const size_t p_h0 = room(split_words(kHeads * kMid, 3, true));
+    size_t p_w2[kHeads], p_w4[kHeads];
+    for (int h = 0; h < kHeads; ++h) {
+        p_w2[h] = room(split1x1_words(kMid));
+        p_w4[h] = room(split1x1_words(kHeadOut[h]));
     }
+    std::vector<float> staging(raw);
+    for (size_t i = 0; i < ns; ++i)
+        std::memcpy(&staging[at[i]], host[i].data(), host[i].size() * sizeof(float));
+    hipError_t e;
     if (!warena) {
-        const hipError_t e = hipMalloc(&warena, total * sizeof(float));
+        e = hipMalloc(&warena, total * sizeof(float));
         if (e != hipSuccess) {
             warena = nullptr;
             return hip_fail(e, "hipMalloc of the weights");
@@ -675,13 +589,43 @@ int bvml_dsine_refiner::upload() {
     } else {
         // a forward queued earlier, on any stream of the device, may still be
         // reading the weights: wait for it before overwriting them
-        const hipError_t e = hipDeviceSynchronize();
+        e = hipDeviceSynchronize();
         if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
     }
-    const hipError_t e = hipMemcpy(warena, staging.data(), total * sizeof(float),
-                                   hipMemcpyHostToDevice);
+    e = hipMemcpy(warena, staging.data(), raw * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "weight upload");
-    for (size_t k = 0; k < parts.size(); ++k) *parts[k].first = warena + offset[k];
+    auto dev = [&](int spec) { return warena + at[spec]; };
+    std::vector<PackArgs> packs;
+    packs.push_back({{dev(kZw), dev(kRw), dev(kQw)}, kHidden, 1, 3 * kHidden, kHx, kHidden, kHx, 5,
+                     warena + p_ctx});
+    packs.push_back({{dev(kZw), dev(kRw)}, kHidden, 1, 2 * kHidden, kHx, 0, kHidden, 5,
+                     warena + p_zr});
+    packs.push_back({{dev(kQw)}, kHidden, 0, kHidden, kHx, 0, kHidden, 5, warena + p_q});
+    PackArgs first{{}, kMid, 0, kHeads * kMid, kHin, 0, kHin, 3, warena + p_h0};
+    for (int h = 0; h < kHeads; ++h) {
+        first.src[h] = dev(head_w(h, 0));
+        packs.push_back({{dev(head_w(h, 1))}, kMid, 0, kMid, kMid, 0, kMid, 1, warena + p_w2[h]});
+        packs.push_back({{dev(head_w(h, 2))}, kHeadOut[h], 0, kHeadOut[h], kMid, 0, kMid, 1,
+                         warena + p_w4[h]});
+    }
+    packs.push_back(first);
+    for (const PackArgs& p : packs)
+        if ((e = kern->pack(p, stream)) != hipSuccess) return hip_fail(e, "weight packing");
+    // (complete before a forward on any other stream reads them)
+    e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
+    w_ctx = warena + p_ctx;
+    w_zr = warena + p_zr;
+    w_q = warena + p_q;
+    w_h0 = warena + p_h0;
+    b_z = dev(kZb);
+    b_r = dev(kRb);
+    b_q = dev(kQb);
+    for (int h = 0; h < kHeads; ++h) {
+        w2[h] = warena + p_w2[h];
+        w4[h] = warena + p_w4[h];
+        for (int l = 0; l < 3; ++l) b_h[h][l] = dev(head_b(h, l));
+    }
     dirty = false;
     return BVML_DSINE_OK;
 }
@@ -727,7 +671,6 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     // the grid-scaled intrinsics (src/dsine_refine.cpp:232-237)
     const double sw = (double)w8 / a.orig_w, sh = (double)h8 / a.orig_h;
     const double fu = a.fx * sw, cu = (a.cx + 0.5) * sw, fv = a.fy * sh, cv = (a.cy + 0.5) * sh;
-    const int C = kHidden;
     auto copy = [&](float* dst, const float* src, size_t planes) {
         return hipMemcpyAsync(dst, src, planes * hw * b, hipMemcpyDeviceToDevice, strm);
     };
@@ -737,66 +680,67 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
                    ? BVML_DSINE_OK
                    : fail(status, std::string("forward: ") + what + ": " + bvml_dsine_last_error());
     };
+    auto hip = [](hipError_t e, const char* what) {
+        return e == hipSuccess ? BVML_DSINE_OK : hip_fail(e, what);
+    };
     hipError_t e;
-    // hx = [h | feature | uv], rh = r*h, hin = [h_new | uv]
-    float* uv = m.hx + (size_t)(kHidden + kFeature) * hw;
-    if ((st = ck(bvml_dsine_build_uv8_f32(uv, fu, cu, fv, cv, h8, w8, stream), "build_uv8")) ||
-        (st = ck(bvml_dsine_build_ray8_f32(m.ray, fu, cu, fv, cv, h8, w8, stream), "build_ray8")))
-        return st;
-    // (h itself is not copied: the first iteration reads the decoder's
-    // hidden state, and its update writes h_new into hx)
-    if ((e = copy(m.hx + (size_t)kHidden * hw, a.feature, kFeature)) != hipSuccess ||
-        (e = copy(m.hin + (size_t)kHidden * hw, uv, 2)) != hipSuccess ||
-        (e = copy(m.pred[0], a.normal, 3)) != hipSuccess)
-        return hip_fail(e, "hipMemcpyAsync");
-    // pred_norm = RayReLU(decoder.normal, ray_8)  (:240-242)
-    if ((st = ck(bvml_dsine_ray_relu_f32(m.pred[0], m.ray, 1, h8, w8, 0, stream), "ray_relu")))
-        return st;
+    const Kernels* kern = kernels();
+    if (!kern) return fail(BVML_DSINE_EUNSUP, "forward: built without the device kernels");
+    // the camera's maps, pred = RayReLU(decoder.normal, ray_8) (:240-242), the
+    // split maps
+    PrologueArgs pa{};
+    pa.normal = a.normal; pa.hidden = a.hidden; pa.feature = a.feature;
+    pa.fu = fu; pa.cu = cu; pa.fv = fv; pa.cv = cv;
+    pa.H = h8; pa.W = w8;
+    pa.ray = m.ray; pa.uv = m.uv; pa.pred = m.pred[0];
+    pa.hf = m.hf; pa.hs = m.hs; pa.fs = m.fs;
+    pa.th = reinterpret_cast<uint32_t*>(m.th); pa.tf = reinterpret_cast<uint32_t*>(m.tf);
+    pa.info = reinterpret_cast<uint32_t*>(m.info);
+    if ((st = hip(kern->prologue(pa, strm), "prologue"))) return st;
     // the ConvGRU convolutions' parts over [feature | uv], which no
     // iteration changes: once per forward instead of once per iteration
-    float* cf_zr = m.cf;
-    float* cf_q = m.cf + (size_t)2 * kHidden * hw;
-    const float* xf = m.hx + (size_t)kHidden * hw;
-    if ((st = ck(bvml_dsine_conv_f32(xf, kX, h8, w8, r->w_zr_f, 2 * kHidden, 5, cf_zr, stream),
-                 "conv")) ||
-        (st = ck(bvml_dsine_conv_f32(xf, kX, h8, w8, r->w_q_f, kHidden, 5, cf_q, stream), "conv")))
-        return st;
+    ConvArgs base{};
+    base.info = pa.info; base.uv = m.uv; base.H = h8; base.W = w8;
+    ConvArgs ctx = base;
+    ctx.xs = m.fs; ctx.x32 = m.fs; ctx.tail = pa.tf; ctx.which = 1;
+    ctx.wp = r->w_ctx; ctx.cout = ctx.wcout = 3 * kHidden; ctx.out = m.cf;
+    if ((st = hip(kern->conv(Conv::Context, ctx, strm), "context convolution"))) return st;
+    // the ConvGRU (:138-159): the 5x5 convolutions over h (r*h) plus their
+    // parts over [feature | uv], with the gates and the update in their
+    // epilogues; h_new goes over h, in c4 and split
+    ConvArgs gates = base;
+    gates.xs = m.hs; gates.x32 = m.hf; gates.wp = r->w_zr; gates.cout = gates.wcout = 2 * kHidden;
+    gates.s0 = m.cf; gates.b0 = r->b_z; gates.b1 = r->b_r; gates.hf = m.hf; gates.z = m.z;
+    gates.rs = m.rs;
+    ConvArgs update = base;
+    update.xs = m.rs; update.x32 = m.rs; update.wp = r->w_q; update.cout = update.wcout = kHidden;
+    update.s0 = m.cf + (size_t)2 * kHidden * hw; update.b0 = r->b_q; update.hf = m.hf;
+    update.z = m.z; update.out = m.hf; update.outs = m.hs;
+    // the heads (:119-127, :257-267, :276): in the first four iterations the
+    // three the propagate reads, in the last all four; the up-mask head's last
+    // bias is the upsample's
+    ConvArgs heads = base;
+    heads.xs = m.hs; heads.x32 = m.hf; heads.tail = pa.th; heads.wp = r->w_h0;
+    heads.wcout = kHeads * kMid;
+    for (int h = 0; h < kHeads; ++h) {
+        heads.w2[h] = r->w2[h];
+        heads.w4[h] = r->w4[h];
+        heads.hb0[h] = r->b_h[h][0];
+        heads.hb2[h] = r->b_h[h][1];
+        heads.b4[h] = h < kHeads - 1 ? r->b_h[h][2] : nullptr;
+        heads.hout[h] = m.head[h];
+        heads.nout[h] = kHeadOut[h];
+    }
 
     const bool direct = pad_t == 0 && pad_l == 0 && out_h == fh && out_w == fw;
     int cur = 0;
     for (int it = 0; it < kIter; ++it) {
         const bool last = it == kIter - 1;
-        const int nh = last ? kHeads : kHeads - 1;
-        // ConvGRU (:138-159): the two 5x5 convolutions over h (r*h) plus
-        // their parts over [feature | uv], with the gates and the update in
-        // their epilogues; h_new goes to hx (over h after the first
-        // iteration, which reads the decoder's hidden state) and into hin
-        const float* h = it == 0 ? a.hidden : m.hx;
-        if ((st = ck(bvml_dsine_conv_gru_gates_sum_f32(h, kHidden, h8, w8, r->w_zr_h, C, cf_zr,
-                                                       r->b_z, r->b_r, h, m.z, m.rh, stream),
-                     "conv_gru_gates")) ||
-            (st = ck(bvml_dsine_conv_gru_update_sum_f32(m.rh, kHidden, h8, w8, r->w_q_h, C, cf_q,
-                                                        r->b_q, m.z, h, m.hx, m.hin, stream),
-                     "conv_gru_update")))
+        heads.cout = (last ? kHeads : kHeads - 1) * kMid;
+        if ((st = hip(kern->conv(Conv::Gates, gates, strm), "gates convolution")) ||
+            (st = hip(kern->conv(Conv::Update, update, strm), "update convolution")) ||
+            (st = hip(kern->conv(Conv::Heads, heads, strm), "heads convolution")))
             return st;
-        // the heads (:119-127, :257-267, :276): in the first four iterations
-        // the three the propagate reads, as their 3x3 layer with the rest in
-        // its epilogue; in the last all four, the 3x3 layers, then the rest
-        // in one pass (the up-mask head's last layer, 576 outputs, is too
-        // large to fuse); the up-mask head's last bias is the upsample's
-        const float* b4[kHeads] = {r->b4[0], r->b4[1], r->b4[2], nullptr};
-        if (!last) {
-            if ((st = ck(bvml_dsine_conv_heads_f32(m.hin, kHin, h8, w8, r->w_h0p[0], nh, r->b_h0,
-                                                   r->w2q, r->b_h2, r->w4p, b4, kHeadOut, m.head,
-                                                   stream), "conv_heads")))
-                return st;
-        } else if ((st = ck(bvml_dsine_conv_f32(m.hin, kHin, h8, w8, r->w_h0p[1], nh * kMid, 3,
-                                                m.t0, stream), "conv")) ||
-                   (st = ck(bvml_dsine_heads_mlp_f32(m.t0, r->b_h0, r->w2p, r->b_h2, r->w4p, b4,
-                                                     kHeadOut, nh, h8, w8, m.head, stream),
-                            "heads_mlp"))) {
-            return st;
-        }
         // the propagate on the logits (:262-274)
         if ((st = ck(bvml_dsine_angmf_propagate_f32(m.pred[cur], m.head[0], m.head[1],
                                                     m.head[2], m.ray, fu, cu, fv, cv, 1, h8, w8,
@@ -809,7 +753,7 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
         if (!last) continue;
         // up_pred_norm = normalize(convex_upsample(pred_norm, up_mask))  (:276-283)
         float* dst = direct ? out : m.up;
-        if ((st = ck(bvml_dsine_convex_upsample_bias_f32(m.pred[cur], m.head[3], r->b4[3], 1, 3,
+        if ((st = ck(bvml_dsine_convex_upsample_bias_f32(m.pred[cur], m.head[3], r->b_h[3][2], 1, 3,
                                                          h8, w8, kUp, 1, kUpEps, dst, 0, stream),
                      "convex_upsample")))
             return st;
@@ -915,7 +859,7 @@ int bvml_dsine_refiner_forward(bvml_dsine_refiner* r, const float* normal, const
     DeviceScope scope(r->device);
     if (scope.status() != hipSuccess) return hip_fail(scope.status(), "hipSetDevice");
     int st;
-    if (r->dirty && (st = r->upload()) != BVML_DSINE_OK) return st;
+    if (r->dirty && (st = r->upload(static_cast<hipStream_t>(stream))) != BVML_DSINE_OK) return st;
     if ((st = r->plan(h8, w8)) != BVML_DSINE_OK) return st;
     return bvml_refine::forward_maps(r, r->maps, args, stream);
 }

@@ -68,31 +68,33 @@ int check_forward(const std::vector<std::vector<float>>& host, const ForwardArgs
 // The host copy of the refiner's weights, one vector per spec.
 const std::vector<std::vector<float>>& host_weights(const bvml_dsine_refiner* r);
 
-// The device maps of one forward: [h | feature | uv], r*h, [h_new | uv], the
-// update gate, the heads' 3x3 output, the heads' outputs, the two propagate
-// buffers, the ray map, the full-resolution result before the crop, and the
+// The device maps of one forward (layouts: refiner_kernels.h): the hidden
+// state (c4 and split), r*h and the features (split), the update gate, the
 // ConvGRU convolutions' parts over [feature | uv] (constant through the
 // iterations: convz + convr's 128 channels in their packed order, then
-// convq's 64).
+// convq's 64), the uv map and the two tails, the heads' outputs, the two
+// propagate buffers, the ray map, the full-resolution result before the crop,
+// the scales.
 struct Maps {
-    float *hx, *rh, *hin, *z, *t0, *head[kHeads], *pred[2], *ray, *up, *cf;
+    float *hf, *hs, *rs, *fs, *z, *cf, *uv, *th, *tf, *head[kHeads], *pred[2], *ray, *up, *info;
 };
 
-// The planes of each map in Maps order (up: 3 * kUp^2 planes); each map
-// starts on a 64-float boundary.
-constexpr int kMapPlanes[] = {kHx, kHidden, kHin, kHidden, kHeads * kMid, kHeadOut[0],
-                              kHeadOut[1], kHeadOut[2], kHeadOut[3], 3, 3, 3, 3 * kUp * kUp,
-                              3 * kHidden};
-inline size_t maps_floats(size_t hw) {
-    size_t total = 0;
+// The planes of each map in Maps order (up: 3 * kUp^2 planes), info apart;
+// each map starts on a 64-float boundary.
+constexpr int kMapPlanes[] = {kHidden, kHidden, kHidden, kFeature, kHidden, 3 * kHidden,
+                              2, 2, 2, kHeadOut[0], kHeadOut[1], kHeadOut[2], kHeadOut[3],
+                              3, 3, 3, 3 * kUp * kUp};
+constexpr size_t kInfoFloats = 64 + 2 * 256;
+constexpr size_t maps_floats(size_t hw) {
+    size_t total = kInfoFloats;
     for (int c : kMapPlanes) total += ((size_t)c * hw + 63) & ~(size_t)63;
     return total;
 }
 inline Maps maps_at(float* base, size_t hw) {
     Maps m{};
-    float** order[] = {&m.hx,      &m.rh,      &m.hin,     &m.z,       &m.t0,
-                       &m.head[0], &m.head[1], &m.head[2], &m.head[3], &m.pred[0],
-                       &m.pred[1], &m.ray,     &m.up,      &m.cf};
+    float** order[] = {&m.hf,      &m.hs,      &m.rs,      &m.fs,      &m.z,       &m.cf,
+                       &m.uv,      &m.th,      &m.tf,      &m.head[0], &m.head[1], &m.head[2],
+                       &m.head[3], &m.pred[0], &m.pred[1], &m.ray,     &m.up};
     static_assert(sizeof(order) / sizeof(order[0]) == sizeof(kMapPlanes) / sizeof(kMapPlanes[0]),
                   "one plane count per map");
     size_t at = 0;
@@ -100,6 +102,7 @@ inline Maps maps_at(float* base, size_t hw) {
         *order[i] = base + at;
         at += ((size_t)kMapPlanes[i] * hw + 63) & ~(size_t)63;
     }
+    m.info = base + at;
     return m;
 }
 

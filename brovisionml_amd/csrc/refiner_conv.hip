@@ -1,0 +1,1033 @@
+// The native refiner's own kernels: its ConvGRU's 5x5 and its heads' 3x3
+// convolutions (stride 1, zero "same" padding) with everything around them
+// fused (src/dsine_refine.cpp:119-159), and the first steps of a forward.
+//
+// The convolutions are implicit GEMMs on the f16 matrix cores at fp32
+// precision.  Every operand, scaled by a power of two, is the sum of two
+// halfs, hi = half(v) and lo = half(v - hi), to within 2^-23 of itself; a
+// product is three matrix-core products (hi hi + hi lo + lo hi; the omitted
+// lo lo is at most 2^-22 of it) summed in fp32.  The weights are split when
+// they are packed, each output channel scaled to its largest weight; a map is
+// split by the kernel that writes it, scaled to a bound of its values: the
+// largest feature, and for the hidden state the largest of 1 and the decoder's
+// |hidden| (a ConvGRU state never exceeds it).  A value is kept to full
+// precision down to 2^-29 of the bound, and none is off by more than 2^-39 of
+// it.  The scales come off the sums exactly.  Where an operand has no such
+// scale (an infinity, a NaN, magnitudes from 2^64) the same kernels convolve
+// the fp32 maps on the fp32 matrix cores.
+//
+// Three v_mfma_f32_16x16x32_f16 (16 cycles each) do the work of eight
+// v_mfma_f32_16x16x4_f32 (32 cycles each), and the sums' chains are shorter
+// (150 additions instead of 400 for 64 channels and 25 taps): relative rms
+// error 4.4e-7 against 7.1e-7 for the fp32 kernel on the same operands.
+
+#include <hip/hip_runtime.h>
+
+#include <climits>
+#include <cstdint>
+
+#include "angmf_ref.h"
+#include "refiner_kernels.h"
+
+namespace {
+
+using namespace bvml_refine;
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTW = 16;  // tile width: one MFMA column block per tile row
+
+constexpr int kMaxOuts = 576;  // a head's outputs
+
+enum Epi : int { kPlain = 0, kGates = 1, kUpdate = 2, kHeads = 3 };
+
+struct KArgs {
+    ConvArgs c;
+    int wblocks, tiles_x, mgroups;
+    uint32_t HW;
+};
+
+__device__ __forceinline__ float relu(float v) { return v < 0.0f ? 0.0f : v; }
+__device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+__device__ __forceinline__ float gru_mix(float z, float h, float q) {
+#pragma clang fp contract(off)
+    const float omz = 1.0f - z;
+    return omz * h + z * q;
+}
+__device__ __forceinline__ uint32_t absbits(float v) {
+    return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+}
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t wave_max(uint32_t m) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) m = umax(m, (uint32_t)__shfl_xor((int)m, d));
+    return m;
+}
+
+constexpr uint32_t kInfBits = 0x7f800000u;
+
+// The power of two that brings a magnitude of these bits into [2^14, 2^15),
+// as its exponent (at most 126, so that it is a normal float: a magnitude
+// below 2^-112 stays smaller).
+__device__ __forceinline__ int scale_exp(uint32_t bits) {
+    const int n = 14 + 127 - (int)(bits >> 23);
+    return n < 126 ? n : 126;
+}
+__device__ __forceinline__ float pow2(int n) {
+    return __builtin_bit_cast(float, (uint32_t)(n + 127) << 23);
+}
+
+template <int N, typename H>
+__device__ __forceinline__ void split_to(const float (&v)[N], H& hi, H& lo) {  // already scaled
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        hi[j] = (_Float16)v[j];
+        lo[j] = (_Float16)(v[j] - (float)hi[j]);
+    }
+}
+
+// Raw buffer loads of packed weights: the descriptor in scalar registers, a
+// per-lane byte offset and a wave-uniform one.
+constexpr int kBufferWord3 = 0x00020000;  // gfx9 raw-buffer descriptor word 3
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const float* w, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w), (short)0, (int)bytes,
+                                             kBufferWord3);
+}
+__device__ __forceinline__ h8 ld16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff) {
+    return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0));
+}
+
+// K: kernel size; TAIL: the two extra channels; each wave MB 16-channel
+// blocks x NB tile rows; WM x WN waves along the channels and the rows; KS
+// groups of those waves that split the reduction's steps; AD: steps whose
+// weights are in flight.
+template <int K_, bool TAIL_, int MB_, int NB_, int WM_, int WN_, int KS_, int AD_, int EPI_>
+struct Shape {
+    static constexpr int K = K_, MB = MB_, NB = NB_, WM = WM_, WN = WN_, KS = KS_, AD = AD_,
+                         EPI = EPI_;
+    static constexpr bool TAIL = TAIL_;
+    static constexpr int kWaves = WM * WN * KS, kThreads = 64 * kWaves;
+    static constexpr int TH = NB * WN;
+    static constexpr int HR = TH + K - 1, HC = kTW + K - 1, HS = HR * HC;
+    // a multiple of 16 pixels: 256 bytes, so the four channel groups that a B
+    // read takes fall on the banks its 16 columns leave free
+    static constexpr int HSP = (HS + 15) / 16 * 16;
+    static constexpr int kHaloBytes = 2 * 8 * HSP * 16;
+    static constexpr int kTailPx = HS + 8;
+    static constexpr int kTailBytes = TAIL ? 2 * kTailPx * 4 : 0;
+    // the groups' partial sums, all but each group's own columns
+    static constexpr int kXchBytes = KS > 1 ? WM * WN * (KS - 1) * MB * NB * 1024 : 0;
+    // the heads' operands and exponents
+    static constexpr int kHeadBytes = EPI == kHeads ? TH * 4416 + 64 + 8 * kMaxOuts : 0;
+    static constexpr int kMainBytes = kHaloBytes + kTailBytes;
+    static constexpr int kLdsBytes = kMainBytes > kXchBytes
+                                         ? (kMainBytes > kHeadBytes ? kMainBytes : kHeadBytes)
+                                         : (kXchBytes > kHeadBytes ? kXchBytes : kHeadBytes);
+    static constexpr int NC = NB >= KS ? NB / KS : 1;  // columns (tile rows) a wave finishes
+    static_assert(NB % KS == 0 || NB < KS, "whole columns per group");
+    static_assert(16 % kWaves == 0, "waves share a halo's 16 planes evenly");
+    static_assert(AD % 2 == 0, "B operands alternate between two slots");
+};
+
+template <class S>
+__global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
+    constexpr int K = S::K, P = K / 2, TAPS = K * K, MAIN = 2 * TAPS;
+    constexpr bool TAIL = S::TAIL;
+    constexpr int STEPS = split_steps(K, TAIL);
+    constexpr int MB = S::MB, NB = S::NB, WM = S::WM, WN = S::WN, KS = S::KS, AD = S::AD;
+    constexpr int HC = S::HC, HS = S::HS, HSP = S::HSP, NC = S::NC, EPI = S::EPI;
+    __shared__ __align__(16) char lds[S::kLdsBytes];
+
+    const ConvArgs& c = a.c;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, col = lane & 15;
+    const int wm = wave % WM, wn = (wave / WM) % WN, ks = wave / (WM * WN);
+    // each XCD takes a contiguous run of (tile, channel group) pairs
+    // (workgroups go to the 8 XCDs in turn), so neighbouring tiles share
+    // their halo lines in one L2
+    const int nbx = (int)gridDim.x, bx = (int)blockIdx.x, xcd = bx & 7;
+    const int id = xcd * (nbx >> 3) + (xcd < (nbx & 7) ? xcd : (nbx & 7)) + (bx >> 3);
+    const int tile = id / a.mgroups, mg = id - tile * a.mgroups;
+    const int tx0 = (tile % a.tiles_x) * kTW, ty0 = (tile / a.tiles_x) * S::TH;
+    const int mb0 = mg * (MB * WM) + MB * wm;  // the wave's first M-block
+    const int H = c.H, W = c.W;
+    const size_t HW = a.HW;
+
+    // the wave's steps of the reduction
+    const int st0 = KS > 1 ? STEPS * ks / KS : 0;
+    const int st1 = KS > 1 ? STEPS * (ks + 1) / KS : STEPS;
+    const int sm1 = st1 < MAIN ? st1 : MAIN;  // (the tail's steps come last)
+
+    const int* const wexp = reinterpret_cast<const int*>(c.wp);
+    const uint32_t whead = split_head_words(a.wblocks);
+    const Info* const info = reinterpret_cast<const Info*>(c.info);
+    const int xn = info->n[c.which];
+    const bool exact = info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
+
+    const __amdgpu_buffer_rsrc_t wr = rsrc_of(c.wp + whead, (uint32_t)a.wblocks * STEPS * 2048u);
+    const uint32_t lane16 = 16u * (uint32_t)lane;
+    h8 aw[AD][MB][2];
+    auto a_load = [&](int st, int slot) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            const uint32_t so = ((uint32_t)(mb0 + m) * STEPS + (uint32_t)st) * 2048u;
+            aw[slot][m][0] = ld16(wr, lane16, so);
+            aw[slot][m][1] = ld16(wr, lane16 + 1024u, so);
+        }
+    };
+
+    v4f acc[MB][NB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+    if (!exact) {
+        // the halo to LDS with direct-to-LDS loads, 16 bytes a lane: each
+        // wave takes 16 / kWaves of the 16 planes (hi, lo x channel group)
+        const char* const xs = static_cast<const char*>(c.xs);
+        constexpr int PPW = 16 / S::kWaves;
+#pragma unroll
+        for (int ch = 0; ch < (HS + 63) / 64; ++ch) {
+            const int px = ch * 64 + lane;
+            const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
+            if (px < HS) {
+                if (y >= 0 && y < H && x >= 0 && x < W) {
+                    const char* src = xs + ((size_t)(wave * PPW) * HW + (uint32_t)(y * W + x)) * 16;
+#pragma unroll
+                    for (int p = 0; p < PPW; ++p)
+                        __builtin_amdgcn_global_load_lds(
+                            static_cast<const void*>(src + (size_t)p * HW * 16),
+                            reinterpret_cast<__attribute__((address_space(3))) void*>(
+                                reinterpret_cast<uintptr_t>(
+                                    lds + ((wave * PPW + p) * HSP + ch * 64) * 16)),
+                            16, 0, 0);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < PPW; ++p)
+                        *reinterpret_cast<v4u*>(lds + ((wave * PPW + p) * HSP + px) * 16) =
+                            v4u{0, 0, 0, 0};
+                }
+            }
+        }
+        // the first steps' weights, in flight beside the halo
+#pragma unroll
+        for (int u = 0; u < AD; ++u) a_load(st0 + u < st1 ? st0 + u : st1 - 1, u);
+        uint32_t* const tl = reinterpret_cast<uint32_t*>(lds + S::kHaloBytes);
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int i = 0; i < (S::kTailPx + S::kThreads - 1) / S::kThreads; ++i) {
+                const int px = tid + i * S::kThreads;
+                const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
+                const bool in = px < HS && y >= 0 && y < H && x >= 0 && x < W;
+                const uint32_t at = in ? (uint32_t)(y * W + x) : 0u;
+                const uint32_t hi = c.tail[at], lo = c.tail[HW + at];
+                if (px < S::kTailPx) {
+                    tl[px] = in ? hi : 0u;
+                    tl[S::kTailPx + px] = in ? lo : 0u;
+                }
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
+        __syncthreads();
+
+        const char* const hb = lds + (g * HSP + wn * NB * HC + col) * 16;
+        h8 bw[2][NB][2];
+        auto b_load = [&](int st, int slot) {
+            const int cc = st >= TAPS ? 1 : 0, tap = st - cc * TAPS;
+            const int off = (cc * 4 * HSP + (tap / K) * HC + tap % K) * 16;
+            const char* p = hb + off;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                bw[slot][n][0] = *reinterpret_cast<const h8*>(p + n * HC * 16);
+                bw[slot][n][1] = *reinterpret_cast<const h8*>(p + (8 * HSP + n * HC) * 16);
+            }
+        };
+        auto products = [&](int as, int bs) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            aw[as][m][p == 0 ? 1 : 0], bw[bs][n][p == 1 ? 1 : 0], acc[m][n], 0, 0,
+                            0);
+        };
+        int st = st0;
+        b_load(st < MAIN ? st : MAIN - 1, 0);
+        for (; st + AD <= sm1; st += AD) {
+#pragma unroll
+            for (int u = 0; u < AD; ++u) {
+                const int nx = st + u + 1;
+                b_load(nx < MAIN ? nx : MAIN - 1, (u + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+                products(u, u & 1);
+                const int na = st + u + AD;
+                a_load(na < st1 ? na : st1 - 1, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the steps left (their weights are in the slots from 0 on)
+#pragma unroll
+        for (int u = 0; u < AD - 1; ++u) {
+            if (st + u < sm1) {
+                const int nx = st + u + 1;
+                b_load(nx < MAIN ? nx : MAIN - 1, (u + 1) & 1);
+                products(u, u & 1);
+            }
+        }
+        if constexpr (TAIL) {
+            // K = 5: two rows of 8 taps per step (5 of them real), K = 3: the
+            // rows of 4 taps (3 real), both channels of a tap together; a
+            // lane's 8 values are 4 taps of one row, at 4 pixels of the tail
+            for (int ts = st0 > MAIN ? st0 : MAIN; ts < st1; ++ts) {
+                a_load(ts, 0);
+                const int t = ts - MAIN;
+                int row = K == 5 ? 2 * t + (g >> 1) : g;
+                row = row < K ? row : K - 1;  // (zero weights there)
+                const int kx = K == 5 ? 4 * (g & 1) : 0;
+                const int at = (wn * NB + row) * HC + col + kx;
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                    v4u hi, lo;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        hi[q] = tl[at + n * HC + q];
+                        lo[q] = tl[S::kTailPx + at + n * HC + q];
+                    }
+                    bw[0][n][0] = __builtin_bit_cast(h8, hi);
+                    bw[0][n][1] = __builtin_bit_cast(h8, lo);
+                }
+                products(0, 0);
+            }
+        }
+    } else {
+        // fp32 products of the c4 map and the unsplit weights: one 16x16x4
+        // step per tap and 4 channels
+        constexpr int GROUPS = split_groups(TAIL);
+        const float* const w32 = c.wp + whead + (size_t)a.wblocks * STEPS * 512;
+        for (int cg = ks; cg < GROUPS; cg += KS) {
+            const bool tail = cg == 16;
+            for (int tap = 0; tap < TAPS; ++tap) {
+                float af[MB];
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+                    af[m] = w32[(((size_t)(mb0 + m) * GROUPS + cg) * TAPS + tap) * 64 + lane];
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                    const int y = ty0 + wn * NB + n + tap / K - P, x = tx0 + col + tap % K - P;
+                    const bool in = y >= 0 && y < H && x >= 0 && x < W && !(tail && g >= 2);
+                    const size_t px = in ? (uint32_t)(y * W + x) : 0u;
+                    const float f = !TAIL || !tail ? c.x32[((size_t)cg * HW + px) * 4 + g]
+                                                   : c.uv[(g < 2 ? g : 0) * HW + px];
+                    const float bf = in ? f : 0.0f;
+#pragma unroll
+                    for (int m = 0; m < MB; ++m)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[m], bf, acc[m][n], 0,
+                                                                        0, 0);
+                }
+            }
+        }
+    }
+
+    // the groups' partial sums meet: group ks finishes columns n = ks, ks + KS, ...
+    v4f own[MB][NC];
+    if constexpr (KS > 1) {
+        __syncthreads();  // every wave is done with the halo
+        v4f* const xch =
+            reinterpret_cast<v4f*>(lds) + (size_t)(wn * WM + wm) * (KS - 1) * MB * NB * 64 + lane;
+        // column n, block m: the partials of the groups that do not own it
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+            if (n % KS != ks) {
+                const int k = ks < n % KS ? ks : ks - 1;
+#pragma unroll
+                for (int m = 0; m < MB; ++m) xch[((n * MB + m) * (KS - 1) + k) * 64] = acc[m][n];
+            }
+        __syncthreads();
+        if (EPI != kHeads && ks >= NB) return;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+            if (n % KS == ks) {
+#pragma unroll
+                for (int m = 0; m < MB; ++m) {
+                    v4f s = acc[m][n];
+#pragma unroll
+                    for (int k = 0; k < KS - 1; ++k) s += xch[((n * MB + m) * (KS - 1) + k) * 64];
+                    own[m][n / KS] = s;
+                }
+            }
+    } else {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) own[m][n] = acc[m][n];
+    }
+
+    // epilogue: lane (g, col), register r of own[m][j] is output channel
+    // 16 (mb0 + m) + 4 g + r (in the packed order) at pixel (row(j), tx0 + col)
+    const int x = tx0 + col;
+    auto row_of = [&](int j) { return ty0 + wn * NB + j * KS + ks; };
+    // the scales come off
+    if (!exact) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = wexp[16 * (mb0 + m) + 4 * g + r] - xn;
+#pragma unroll
+                for (int j = 0; j < NC; ++j) own[m][j][r] = ldexpf(own[m][j][r], e);
+            }
+    }
+    // channels 16 q + 4 g .. + 3 of a pixel, in c4 and in a split map
+    auto c4_at = [&](int q, uint32_t px) { return ((size_t)(4 * q + g) * HW + px) * 4; };
+    auto store_split = [&](void* base, int q, uint32_t px, const v4f& v) {
+        float s[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[r] = v[r] * pow2(xn);
+        h4 hi, lo;
+        split_to(s, hi, lo);
+        char* p = static_cast<char*>(base) + ((size_t)(2 * q + (g >> 1)) * HW + px) * 16 + 8 * (g & 1);
+        *reinterpret_cast<h4*>(p) = hi;
+        *reinterpret_cast<h4*>(p + 8 * HW * 16) = lo;
+    };
+
+    if constexpr (EPI == kHeads) {
+        // The rest of head mg on the matrix cores, the workgroup's waves
+        // sharing the tile's activations through LDS as operands:
+        //   a = relu(s + b0);  t = relu(W2 a + b2);  out = W4 t + b4.
+        // A 1x1 layer's reduction step of 32 channels takes M-blocks 2q and
+        // 2q + 1: lane (g, col) holds their channels 16 m + 4 g + r, which is
+        // its B operand, the weights being packed in that channel order.  Each
+        // pixel's channels are scaled to their largest and split.  (Each wave
+        // running both layers for its own columns took 107 us for the three
+        // heads at 256 x 256 and 405 us for all four: every wave streamed
+        // every weight, one load's latency per 16 outputs.)
+        static_assert(EPI != kHeads || (MB == 4 && WM == 1), "one head per wave");
+        static_assert(EPI != kHeads || (S::kWaves % 4 == 0 && S::TH % (S::kWaves / 4) == 0 &&
+                                        S::TH % 2 == 0), "the waves share the layers");
+        constexpr int TH = S::TH;
+        // LDS: the operands [q 0, 1][hi, lo][row][lane] 16 bytes (or the fp32
+        // activations [m][row][lane], where one is infinite or NaN), each
+        // pixel's exponent in the first layer, its largest t per M-block, the
+        // waves' largest, the last layer's exponents and biases
+        char* const frag = lds;
+        int* const e1 = reinterpret_cast<int*>(lds + TH * 4096);
+        uint32_t* const pm = reinterpret_cast<uint32_t*>(lds + TH * 4096 + TH * 64);
+        uint32_t* const red = reinterpret_cast<uint32_t*>(lds + TH * 4096 + TH * 320);
+        int* const e4s = reinterpret_cast<int*>(lds + TH * 4416 + 64);
+        float* const b4s = reinterpret_cast<float*>(e4s + kMaxOuts);
+        const int hd = mg;
+        const float* w2 = c.w2[hd];
+        const float* w4 = c.w4[hd];
+        const float* b4 = c.b4[hd];
+        float* out = c.hout[hd];
+        const int nout = c.nout[hd], nob = (nout + 15) / 16;
+        constexpr uint32_t kHead64 = split1x1_head_words(64);
+        const uint32_t head4 = split1x1_head_words(nout);
+        const __amdgpu_buffer_rsrc_t r2 = rsrc_of(w2 + kHead64, 4 * 2 * 2048u);
+        const __amdgpu_buffer_rsrc_t r4 = rsrc_of(w4 + head4, (uint32_t)nob * 2 * 2048u);
+        const int* e2 = reinterpret_cast<const int*>(w2);
+        const int* e4 = reinterpret_cast<const int*>(w4);
+        const bool ok2 = e2[64] != 0, ok4 = e4[16 * nob] != 0;
+        auto w_load = [&](__amdgpu_buffer_rsrc_t rr, int ob, h8 (&w)[2][2]) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                w[q][0] = ld16(rr, lane16, (uint32_t)(ob * 2 + q) * 2048u);
+                w[q][1] = ld16(rr, lane16 + 1024u, (uint32_t)(ob * 2 + q) * 2048u);
+            }
+        };
+        auto frag_at = [&](int q, int hl, int row) {
+            return reinterpret_cast<h8*>(frag + (((q * 2 + hl) * TH + row) * 64 + lane) * 16);
+        };
+        auto act_at = [&](int m, int row) {
+            return reinterpret_cast<v4f*>(frag + ((m * TH + row) * 64 + lane) * 16);
+        };
+        // 16 outputs for one row of pixels, split and fp32
+        auto split16 = [&](const h8 (&w)[2][2], const h8 (&b)[2][2], v4f o) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    o = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[q][p == 0 ? 1 : 0],
+                                                               b[q][p == 1 ? 1 : 0], o, 0, 0, 0);
+            return o;
+        };
+        auto exact16 = [&](const float* w32, int ob, int row) {
+            v4f o = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int m = 0; m < 4; ++m) {
+                const v4f v = *act_at(m, row);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    o = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        w32[((size_t)ob * 16 + 4 * m + r) * 64 + lane], v[r], o, 0, 0, 0);
+            }
+            return o;
+        };
+
+        h8 wa[2][2];
+        const int mo = wave & 3;  // the wave's M-block of t
+        w_load(r2, mo, wa);
+        // a of the wave's own columns, and their pixels' largest
+        uint32_t mx[NC], top = 0;
+        if (ks < NB) {
+            v4f b0v[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                b0v[m] = *reinterpret_cast<const v4f*>(c.hb0[hd] + 16 * m + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                mx[j] = 0;
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        own[m][j][r] = relu(own[m][j][r] + b0v[m][r]);
+                        mx[j] = umax(mx[j], absbits(own[m][j][r]));
+                    }
+                mx[j] = umax(mx[j], (uint32_t)__shfl_xor((int)mx[j], 16));
+                mx[j] = umax(mx[j], (uint32_t)__shfl_xor((int)mx[j], 32));
+                top = umax(top, mx[j]);
+            }
+        }
+        __syncthreads();  // the partial sums are read
+        for (int i = tid; i < 16 * nob; i += S::kThreads) {
+            e4s[i] = e4[i];
+            b4s[i] = b4 && i < nout ? b4[i] : 0.0f;
+        }
+        top = wave_max(top);
+        if (lane == 0) red[wave] = top;
+        __syncthreads();
+        bool ok = ok2;
+#pragma unroll
+        for (int w = 0; w < S::kWaves; ++w) ok = ok && red[w] < kInfBits;
+        if (ks < NB) {
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int row = wn * NB + j * KS + ks;
+                if (ok) {
+                    const int n = scale_exp(mx[j]);
+                    const float sc = pow2(n);
+                    if (g == 0) e1[row * 16 + col] = -n;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        float s[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) s[i] = own[2 * q + (i >> 2)][j][i & 3] * sc;
+                        h8 hi, lo;
+                        split_to(s, hi, lo);
+                        *frag_at(q, 0, row) = hi;
+                        *frag_at(q, 1, row) = lo;
+                    }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) *act_at(m, row) = own[m][j];
+                }
+            }
+        }
+        __syncthreads();
+        // t = relu(W2 a + b2): M-block mo of the rows of the wave's share
+        constexpr int R1 = TH / (S::kWaves / 4);
+        const int row1 = (wave >> 2) * R1;
+        v4f t[R1];
+        uint32_t tm[R1];
+        {
+            const v4f b2v = *reinterpret_cast<const v4f*>(c.hb2[hd] + 16 * mo + 4 * g);
+            int ew[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ew[r] = e2[16 * mo + 4 * g + r];
+            top = 0;
+#pragma unroll
+            for (int j = 0; j < R1; ++j) {
+                const int row = row1 + j;
+                v4f o;
+                if (ok) {
+                    h8 b[2][2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        b[q][0] = *frag_at(q, 0, row);
+                        b[q][1] = *frag_at(q, 1, row);
+                    }
+                    o = split16(wa, b, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+                    const int ex = e1[row * 16 + col];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[r] = ldexpf(o[r], ew[r] + ex);
+                } else {
+                    o = exact16(w2 + kHead64 + 4096, mo, row);
+                }
+                tm[j] = 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    t[j][r] = relu(o[r] + b2v[r]);
+                    tm[j] = umax(tm[j], absbits(t[j][r]));
+                }
+                tm[j] = umax(tm[j], (uint32_t)__shfl_xor((int)tm[j], 16));
+                tm[j] = umax(tm[j], (uint32_t)__shfl_xor((int)tm[j], 32));
+                if (g == 0) pm[(mo * TH + row) * 16 + col] = tm[j];
+                top = umax(top, tm[j]);
+            }
+        }
+        top = wave_max(top);
+        __syncthreads();  // a is read
+        if (lane == 0) red[wave] = top;
+        // the last layer's first weights: block `wave / 2` and on, by kWaves / 2
+        constexpr int OBS = S::kWaves / 2;
+        const int ob0 = wave >> 1;
+        if (ok4) w_load(r4, ob0 < nob ? ob0 : nob - 1, wa);
+        __syncthreads();
+        ok = ok4;
+#pragma unroll
+        for (int w = 0; w < S::kWaves; ++w) ok = ok && red[w] < kInfBits;
+        auto px_exp = [&](int row) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) m = umax(m, pm[(k * TH + row) * 16 + col]);
+            return scale_exp(m);
+        };
+#pragma unroll
+        for (int j = 0; j < R1; ++j) {
+            const int row = row1 + j;
+            if (ok) {
+                const float sc = pow2(px_exp(row));
+                float s[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[r] = t[j][r] * sc;
+                h4 hi, lo;
+                split_to(s, hi, lo);
+                reinterpret_cast<h4*>(frag_at(mo >> 1, 0, row))[mo & 1] = hi;
+                reinterpret_cast<h4*>(frag_at(mo >> 1, 1, row))[mo & 1] = lo;
+            } else {
+                *act_at(mo, row) = t[j];
+            }
+        }
+        __syncthreads();
+        // out = W4 t + b4: a wave takes one half of the rows and every OBS-th
+        // block of 16 outputs, its operands in registers
+        constexpr int R2 = TH / 2;
+        const int row2 = (wave & 1) * R2;
+        h8 b[R2][2][2];
+        int ex[R2];
+        if (ok) {
+#pragma unroll
+            for (int j = 0; j < R2; ++j) {
+                ex[j] = -px_exp(row2 + j);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    b[j][q][0] = *frag_at(q, 0, row2 + j);
+                    b[j][q][1] = *frag_at(q, 1, row2 + j);
+                }
+            }
+        }
+        // (The loop's only loads are the weights, issued before the stores of
+        // the block before; the stores are buffer stores, dropped beyond the
+        // map by their offset, not by a branch, so that their count is known:
+        // loads and stores share one counter, and with the exponents and
+        // biases loaded here each block waited for the last one's stores, 458
+        // us for the four heads at 256 x 256.)
+        uint32_t at[R2];
+#pragma unroll
+        for (int j = 0; j < R2; ++j) {
+            const int y = ty0 + row2 + j;
+            at[j] = x < W && y < H ? 4u * (uint32_t)(4 * g * a.HW + y * W + x) : 0xf0000000u;
+        }
+        auto store16 = [&](int ob, const v4f (&o)[R2]) {
+            const int left = nout - 16 * ob;
+            const __amdgpu_buffer_rsrc_t ro =
+                rsrc_of(out + (size_t)16 * ob * HW, (uint32_t)(left < 16 ? left : 16) * a.HW * 4u);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float bias = b4s[16 * ob + 4 * g + r];
+#pragma unroll
+                for (int j = 0; j < R2; ++j)
+                    __builtin_amdgcn_raw_buffer_store_b32(
+                        __builtin_bit_cast(uint32_t, b4 ? o[j][r] + bias : o[j][r]), ro,
+                        (int)(at[j] + (uint32_t)r * 4u * a.HW), 0, 0);
+            }
+        };
+        if (ok) {
+            auto block = [&](int ob) {
+                v4f o[R2];
+#pragma unroll
+                for (int j = 0; j < R2; ++j)
+                    o[j] = split16(wa, b[j], v4f{0.0f, 0.0f, 0.0f, 0.0f});
+                __builtin_amdgcn_sched_barrier(0);
+                w_load(r4, ob + OBS < nob ? ob + OBS : ob, wa);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int ew = e4s[16 * ob + 4 * g + r];
+#pragma unroll
+                    for (int j = 0; j < R2; ++j) o[j][r] = ldexpf(o[j][r], ew + ex[j]);
+                }
+                store16(ob, o);
+            };
+            // (the first block apart: at the loop's head the weights are then
+            // always followed by one block's stores, which their wait leaves
+            // in flight)
+            if (ob0 < nob) {
+                block(ob0);
+                for (int ob = ob0 + OBS; ob < nob; ob += OBS) block(ob);
+            }
+        } else {
+            for (int ob = ob0; ob < nob; ob += OBS) {
+                v4f o[R2];
+#pragma unroll
+                for (int j = 0; j < R2; ++j)
+                    o[j] = exact16(w4 + head4 + (size_t)nob * 1024, ob, row2 + j);
+                store16(ob, o);
+            }
+        }
+    } else if constexpr (EPI == kPlain) {
+        if (x >= W) return;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int y = row_of(j);
+            if (y >= H) continue;
+#pragma unroll
+            for (int m = 0; m < MB; ++m)
+                *reinterpret_cast<v4f*>(c.out + c4_at(mb0 + m, (uint32_t)(y * W + x))) = own[m][j];
+        }
+    } else if constexpr (EPI == kGates) {
+        // M-blocks alternate z, r: block 2i holds z channels 16 i.., 2i + 1
+        // the r channels 16 i..; every load goes out before the first store
+        // (the compiler cannot know that they do not overlap)
+        constexpr int MP = MB / 2;
+        static_assert(EPI != kGates || MB % 2 == 0, "z and r blocks in pairs");
+        if (x >= W) return;
+        const int q0 = mb0 / 2;
+        v4f sz[NC][MP], sr[NC][MP], hv[NC][MP], bz[MP], br[MP];
+#pragma unroll
+        for (int p = 0; p < MP; ++p) {
+            bz[p] = *reinterpret_cast<const v4f*>(c.b0 + 16 * (q0 + p) + 4 * g);
+            br[p] = *reinterpret_cast<const v4f*>(c.b1 + 16 * (q0 + p) + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int y = row_of(j) < H ? row_of(j) : H - 1;
+                const uint32_t px = (uint32_t)(y * W + x);
+                sz[j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p, px));
+                sr[j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p + 1, px));
+                hv[j][p] = *reinterpret_cast<const v4f*>(c.hf + c4_at(q0 + p, px));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int y = row_of(j);
+            if (y >= H) continue;
+            const uint32_t px = (uint32_t)(y * W + x);
+#pragma unroll
+            for (int p = 0; p < MP; ++p) {
+                v4f zz, rh;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    zz[r] = sigmoid(own[2 * p][j][r] + sz[j][p][r] + bz[p][r]);
+                    rh[r] = sigmoid(own[2 * p + 1][j][r] + sr[j][p][r] + br[p][r]) * hv[j][p][r];
+                }
+                *reinterpret_cast<v4f*>(c.z + c4_at(q0 + p, px)) = zz;
+                if (info->exact[0])
+                    *reinterpret_cast<v4f*>(static_cast<float*>(c.rs) + c4_at(q0 + p, px)) = rh;
+                else
+                    store_split(c.rs, q0 + p, px, rh);
+            }
+        }
+    } else {
+        if (x >= W) return;
+        v4f bq[MB], sq[NC][MB], zv[NC][MB], hv[NC][MB];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            bq[m] = *reinterpret_cast<const v4f*>(c.b0 + 16 * (mb0 + m) + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int y = row_of(j) < H ? row_of(j) : H - 1;
+                const size_t at = c4_at(mb0 + m, (uint32_t)(y * W + x));
+                sq[j][m] = *reinterpret_cast<const v4f*>(c.s0 + at);
+                zv[j][m] = *reinterpret_cast<const v4f*>(c.z + at);
+                hv[j][m] = *reinterpret_cast<const v4f*>(c.hf + at);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int y = row_of(j);
+            if (y >= H) continue;
+            const uint32_t px = (uint32_t)(y * W + x);
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+                v4f hn;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    hn[r] = gru_mix(zv[j][m][r], hv[j][m][r],
+                                    tanhf(own[m][j][r] + sq[j][m][r] + bq[m][r]));
+                *reinterpret_cast<v4f*>(c.out + c4_at(mb0 + m, px)) = hn;
+                if (!info->exact[0]) store_split(c.outs, mb0 + m, px, hn);
+            }
+        }
+    }
+}
+
+template <class S>
+hipError_t launch(const ConvArgs& c, hipStream_t stream) {
+    KArgs a{};
+    a.c = c;
+    a.wblocks = c.wcout / 16;
+    a.HW = (uint32_t)((size_t)c.H * c.W);
+    a.tiles_x = (c.W + kTW - 1) / kTW;
+    a.mgroups = c.cout / (16 * S::MB * S::WM);
+    const long long groups =
+        (long long)a.tiles_x * ((c.H + S::TH - 1) / S::TH) * a.mgroups;
+    if (groups > INT_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((conv_kernel<S>), dim3((unsigned)groups), dim3(S::kThreads), 0, stream, a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Packing the weights: a workgroup per 16-channel block.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
+    const int mb = (int)blockIdx.x, nmb = (int)gridDim.x, taps = a.k * a.k, tid = (int)threadIdx.x;
+    const bool one = a.k == 1;
+    const int cin = a.c1 - a.c0, cols = cin * taps;
+    const size_t stride = (size_t)a.cin * taps;  // of a source row
+    __shared__ uint32_t rowmax[16];
+    __shared__ const float* rowp[16];
+    if (tid < 16) {
+        rowmax[tid] = 0;
+        const int o = 16 * mb + tid;
+        int blk = 0, within = o;
+        if (a.interleave) {
+            blk = (o >> 4) & 1;
+            within = 16 * (o >> 5) + (o & 15);
+            if (o >= 32 * (a.rows / 16)) { blk = 2; within = o - 2 * a.rows; }
+        } else {
+            while (blk < 3 && within >= a.rows) { within -= a.rows; ++blk; }
+        }
+        rowp[tid] = o < a.out ? a.src[blk] + (size_t)within * stride + (size_t)a.c0 * taps : nullptr;
+    }
+    __syncthreads();
+    for (int i = tid; i < 16 * cols; i += 256) {
+        const int r = i / cols;
+        if (rowp[r]) atomicMax(&rowmax[r], absbits(rowp[r][i - r * cols]));
+    }
+    __syncthreads();
+    // [exponents | flag], the flag cleared by any block that finds an infinity
+    // or a NaN (it is set before these launches)
+    int* const head = reinterpret_cast<int*>(a.wp);
+    if (tid < 16) {
+        const uint32_t m = rowmax[tid];
+        head[16 * mb + tid] = m < kInfBits ? -scale_exp(m) : 0;
+        if (m >= kInfBits) head[16 * nmb] = 0;
+    }
+    const bool tail = cin > 64;
+    const int steps = one ? 2 : split_steps(a.k, tail);
+    uint16_t* sw = reinterpret_cast<uint16_t*>(a.wp + split_head_words(nmb)) + (size_t)mb * steps * 1024;
+    for (int i = tid; i < steps * 512; i += 256) {
+        const int st = i >> 9, l = (i >> 3) & 63, j = i & 7, g = l >> 4;
+        const float* row = rowp[l & 15];
+        int at = -1;  // the value's place in the row
+        if (one) {
+            at = 16 * (2 * st + j / 4) + 4 * g + j % 4;
+        } else if (st < 2 * taps) {
+            at = (32 * (st / taps) + 8 * g + j) * taps + st % taps;
+        } else {
+            const int t = st - 2 * taps;
+            const int ky = a.k == 5 ? 2 * t + (g >> 1) : g;
+            const int kx = (a.k == 5 ? 4 * (g & 1) : 0) + j / 2;
+            if (ky < a.k && kx < a.k) at = (64 + j % 2) * taps + ky * a.k + kx;
+        }
+        const uint32_t m = rowmax[l & 15];
+        float v[1] = {row && at >= 0 && m < kInfBits ? row[at] * pow2(scale_exp(m)) : 0.0f};
+        typedef _Float16 h1 __attribute__((ext_vector_type(1)));
+        h1 hi, lo;
+        split_to(v, hi, lo);
+        sw[st * 1024 + l * 8 + j] = __builtin_bit_cast(uint16_t, hi);
+        sw[st * 1024 + 512 + l * 8 + j] = __builtin_bit_cast(uint16_t, lo);
+    }
+    float* w32 = a.wp + split_head_words(nmb) + (size_t)nmb * steps * 512;
+    const int groups = one ? 16 : split_groups(tail);
+    w32 += (size_t)mb * groups * taps * 64;
+    for (int i = tid; i < groups * taps * 64; i += 256) {
+        const int l = i & 63, t = (i >> 6) % taps, cg = (i >> 6) / taps;
+        // (a 1x1 layer's step cg = 4 m + r takes inputs 16 m + 4 g + r)
+        const int ch = one ? 16 * (cg >> 2) + 4 * (l >> 4) + (cg & 3) : 4 * cg + (l >> 4);
+        const float* row = rowp[l & 15];
+        w32[i] = row && ch < cin ? row[ch * taps + t] : 0.0f;
+    }
+}
+
+__global__ void pack_flag_kernel(float* wp, int nmb) { reinterpret_cast<int*>(wp)[16 * nmb] = 1; }
+
+hipError_t pack(const PackArgs& a, hipStream_t stream) {
+    const int nmb = (a.out + 15) / 16;
+    hipLaunchKernelGGL(pack_flag_kernel, dim3(1), dim3(1), 0, stream, a.wp, nmb);
+    hipLaunchKernelGGL(pack_kernel, dim3((unsigned)nmb), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// The first steps of a forward, two launches: the maps of the camera, RayReLU
+// of the decoder's normals and the maps' largest magnitudes; then the scales
+// from those and the split maps.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kExactBits = 0x5f800000u;  // 2^64
+
+__global__ __launch_bounds__(256) void camera_kernel(PrologueArgs a, bool vec4) {
+    const uint32_t HW = (uint32_t)a.H * (uint32_t)a.W;
+    const uint32_t tid = blockIdx.x * 256u + threadIdx.x, nt = gridDim.x * 256u;
+    __shared__ uint32_t red[2][4];
+    uint32_t mx[2] = {0, 0};
+    for (int k = 0; k < 2; ++k) {
+        const float* src = k == 0 ? a.hidden : a.feature;
+        const size_t n = (size_t)64 * HW;
+        if (vec4) {
+            for (size_t i = tid; i < n / 4; i += nt) {
+                const v4f v = reinterpret_cast<const v4f*>(src)[i];
+                mx[k] = umax(umax(mx[k], absbits(v[0])), umax(absbits(v[1]), umax(absbits(v[2]), absbits(v[3]))));
+            }
+        } else {
+            for (size_t i = tid; i < n; i += nt) mx[k] = umax(mx[k], absbits(src[i]));
+        }
+    }
+    for (uint32_t p = tid; p < HW; p += nt) {
+        const int y = (int)(p / (uint32_t)a.W), x = (int)(p - (uint32_t)y * a.W);
+        const bvml::Ray3f r = bvml::synth_ray(x, y, a.fu, a.cu, a.fv, a.cv);
+        a.ray[p] = r.x;
+        a.ray[HW + p] = r.y;
+        a.ray[(size_t)2 * HW + p] = r.z;
+        a.uv[p] = (float)(((x + 0.5) - a.cu) / a.fu);
+        a.uv[HW + p] = (float)(((y + 0.5) - a.cv) / a.fv);
+        double ox, oy, oz, inv;
+        bvml::ray_relu_ref(a.normal[p], a.normal[HW + p], a.normal[(size_t)2 * HW + p], r.x, r.y,
+                           r.z, ox, oy, oz, inv);
+        a.pred[p] = (float)ox;
+        a.pred[HW + p] = (float)oy;
+        a.pred[(size_t)2 * HW + p] = (float)oz;
+    }
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t m = wave_max(mx[k]);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const uint32_t* r = red[threadIdx.x];
+        a.info[64 + threadIdx.x * kMaxBlocks + blockIdx.x] =
+            umax(umax(r[0], r[1]), umax(r[2], r[3]));
+    }
+}
+
+// blockIdx.y: 0 hidden, 1 feature (a thread per 8 channels of a pixel), 2 the
+// tails (a thread per pixel).  `blocks`: camera_kernel's; uvmax: the largest
+// |u|, |v| of the map.
+__global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, float uvmax) {
+    const uint32_t HW = (uint32_t)a.H * (uint32_t)a.W;
+    __shared__ uint32_t red[2][4];
+    uint32_t mx[2];
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t m = wave_max(
+            (int)threadIdx.x < blocks ? a.info[64 + k * kMaxBlocks + threadIdx.x] : 0u);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = m;
+    }
+    __syncthreads();
+    int n[2], exact[2];
+    for (int k = 0; k < 2; ++k) {
+        mx[k] = umax(umax(red[k][0], red[k][1]), umax(red[k][2], red[k][3]));
+        const uint32_t one = absbits(1.0f);
+        const uint32_t scale = umax(k == 0 ? umax(mx[k], one) : mx[k], absbits(uvmax));
+        n[k] = scale_exp(scale);
+        // (a uv map far beyond the maps it joins would take their precision)
+        exact[k] = mx[k] >= kExactBits ||
+                   !(uvmax <= 64.0f * __builtin_bit_cast(float, umax(mx[k], one)));
+    }
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        Info* info = reinterpret_cast<Info*>(a.info);
+        for (int k = 0; k < 2; ++k) {
+            info->n[k] = n[k];
+            info->exact[k] = exact[k];
+        }
+    }
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (blockIdx.y == 2) {
+        if (i >= HW) return;
+        for (int k = 0; k < 2; ++k) {
+            uint32_t* t = k == 0 ? a.th : a.tf;
+            const int y = (int)(i / (uint32_t)a.W), x = (int)(i - (uint32_t)y * a.W);
+            const float s[2] = {(float)(((x + 0.5) - a.cu) / a.fu) * pow2(n[k]),
+                                (float)(((y + 0.5) - a.cv) / a.fv) * pow2(n[k])};
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            h2 hi, lo;
+            split_to(s, hi, lo);
+            t[i] = __builtin_bit_cast(uint32_t, hi);
+            t[HW + i] = __builtin_bit_cast(uint32_t, lo);
+        }
+        return;
+    }
+    const uint32_t grp = i / HW, px = i - grp * HW;
+    if (grp >= 8) return;
+    const int k = blockIdx.y;
+    const float* src = (k == 0 ? a.hidden : a.feature) + (size_t)8 * grp * HW + px;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = src[(size_t)j * HW];
+    float* c4 = k == 0 ? a.hf : (exact[1] ? a.fs : nullptr);
+    if (c4) {
+        v4f* d = reinterpret_cast<v4f*>(c4);
+        d[(size_t)(2 * grp) * HW + px] = v4f{v[0], v[1], v[2], v[3]};
+        d[(size_t)(2 * grp + 1) * HW + px] = v4f{v[4], v[5], v[6], v[7]};
+    }
+    if (exact[k]) return;
+    const float sc = pow2(n[k]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= sc;
+    h8 hi, lo;
+    split_to(v, hi, lo);
+    h8* d = reinterpret_cast<h8*>(k == 0 ? a.hs : a.fs);
+    d[(size_t)grp * HW + px] = hi;
+    d[(size_t)(8 + grp) * HW + px] = lo;
+}
+
+hipError_t prologue(const PrologueArgs& a, hipStream_t stream) {
+    const size_t hw = (size_t)a.H * a.W;
+    const size_t want = (hw * 16 + 255) / 256;  // 4 of the 64 channels a thread
+    const int blocks = (int)(want < 1 ? 1 : want > kMaxBlocks ? kMaxBlocks : want);
+    const bool vec4 = ((reinterpret_cast<uintptr_t>(a.hidden) |
+                        reinterpret_cast<uintptr_t>(a.feature)) & 15u) == 0;
+    hipLaunchKernelGGL(camera_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a, vec4);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    auto big = [](double p, double q) { return p > q || p != p ? p : q; };
+    const double uvmax =
+        big(big(std::fabs((0.5 - a.cu) / a.fu), std::fabs((a.W - 0.5 - a.cu) / a.fu)),
+            big(std::fabs((0.5 - a.cv) / a.fv), std::fabs((a.H - 0.5 - a.cv) / a.fv)));
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((8 * hw + 255) / 256), 3), dim3(256), 0,
+                       stream, a, blocks, (float)uvmax);
+    return hipGetLastError();
+}
+
+//           K  TAIL  MB NB WM WN KS AD EPI
+hipError_t conv(Conv op, const ConvArgs& c, hipStream_t stream) {
+    const long long px = (long long)c.H * c.W;
+    switch (op) {
+        case Conv::Context:
+            if (px < 20000) return launch<Shape<5, true, 4, 4, 1, 1, 4, 2, kPlain>>(c, stream);
+            return launch<Shape<5, true, 2, 4, 2, 2, 1, 2, kPlain>>(c, stream);
+        case Conv::Gates:
+            if (px < 20000) return launch<Shape<5, false, 2, 4, 1, 1, 4, 4, kGates>>(c, stream);
+            return launch<Shape<5, false, 4, 4, 2, 4, 1, 2, kGates>>(c, stream);
+        case Conv::Update:
+            if (px < 20000) return launch<Shape<5, false, 2, 4, 1, 1, 4, 4, kUpdate>>(c, stream);
+            return launch<Shape<5, false, 2, 4, 2, 2, 1, 2, kUpdate>>(c, stream);
+        default:
+            if (px < 20000) return launch<Shape<3, true, 4, 4, 1, 1, 4, 2, kHeads>>(c, stream);
+            return launch<Shape<3, true, 4, 4, 1, 2, 2, 2, kHeads>>(c, stream);
+    }
+}
+
+constexpr Kernels kTable = {pack, prologue, conv};
+struct Register {
+    Register() { kernels() = &kTable; }
+} const g_register;
+
+}  // namespace

@@ -24,10 +24,9 @@ namespace {
 
 using namespace bvml_refine;
 
-// 32 MiB: the maps of a grid of up to 5,086 pixels (1,649 planes per
-// pixel; a 60 x 80 grid, the refiner's size for a 480 x 640 image, needs
-// 7,915,200 floats).
-constexpr size_t kScratchFloats = size_t(8) << 20;
+// The maps of a grid of up to 5,086 pixels (a 60 x 80 grid, the refiner's
+// size for a 480 x 640 image, is 4,800), 28 MB.
+constexpr size_t kScratchFloats = maps_floats(5086);
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 constexpr int kMaxDevices = 64;

@@ -1,0 +1,75 @@
+"""The native refiner's own convolutions (brovisionml_amd/csrc/refiner_conv.hip:
+split-half matrix products at fp32 precision) against the float64 restatement
+(oracle/refiner.py), where their tiling, their scales and their fp32 path can
+go wrong: grids around the tile sizes, one-pixel grids, hidden states far from
+unit scale, a field of view whose uv map leaves the split form's range, an
+infinity or a NaN in the decoder's maps.  The bars are those of
+tests/test_gpu_refiner_native.py; a map with a non-finite value has the
+restatement's NaN pattern and its values elsewhere."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from brovisionml_amd import refiner as rf, workloads as wl
+from oracle import refiner as oref
+from tests import refiner_pins as pins
+
+pytestmark = pytest.mark.gpu
+TOL_RESULT, TOL_COARSE = 5e-6, 1e-4
+
+
+def run(H, W, fov, seed, change=None):
+    """(native result, coarse), (restatement's result, coarse)."""
+    import torch
+    print(f"[gpu] refiner {H}x{W} fov {fov}", flush=True)
+    weights = rf.random_weights(seed)
+    maps = [a.copy() for a in pins.inputs(H, W, seed)]
+    if change:
+        change(maps)
+    intr = wl.intrins_from_fov(8 * H, 8 * W, fov)
+    dec = rf.DecoderOutput(*(torch.from_numpy(a)[None].to("cuda:0") for a in maps))
+    out, coarse = rf.NativeRefiner(weights).forward(dec, intr, 8 * H, 8 * W, coarse=True)
+    torch.cuda.synchronize()
+    want = []
+    with np.errstate(all="ignore"):
+        oref.refine_forward(weights, *maps, intr, wl.scaled_intrinsics(intr, H, W, 8 * H, 8 * W),
+                            wl.build_ray8(intr, H, W, 8 * H, 8 * W).reshape(3, H, W),
+                            rf.uv_map(intr, H, W, 8 * H, 8 * W), trace=want, nthreads=16)
+    return ((out.cpu().numpy()[0].astype(np.float64), coarse.cpu().numpy().astype(np.float64)),
+            (want[-1][1], np.stack([c.reshape(3, H, W) for c, _ in want])))
+
+
+def check(got, want, grow=1.0):
+    """grow: how much larger the convolutions' sums, and so their rounding,
+    are than for maps of unit scale (at most the maps' own scale)."""
+    for g, w, tol in ((got[0], want[0], TOL_RESULT), (got[1], want[1], TOL_COARSE)):
+        assert np.array_equal(np.isnan(g), np.isnan(w))
+        err = np.nanmax(np.abs(g - w), initial=0.0)
+        print(f"    max-abs {err:.3e}, {np.isnan(w).mean():.3f} NaN", flush=True)
+        assert err <= grow * tol
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (1, 33), (2, 16), (3, 17), (4, 15), (9, 31), (8, 48),
+                                 (17, 65), (129, 161)])
+def test_grids(cuda, H, W):
+    check(*run(H, W, 60.0, H + W))
+
+
+@pytest.mark.parametrize("scale", [1e-6, 30.0])
+def test_hidden_scale(cuda, scale):
+    def change(maps):
+        maps[2] *= np.float32(scale)
+    check(*run(13, 24, 60.0, 31, change), grow=max(1.0, scale))
+
+
+def test_wide_field_of_view(cuda):
+    """u reaches 572: the maps go through the fp32 products."""
+    check(*run(13, 24, 179.8, 37), grow=572.0)
+
+
+@pytest.mark.parametrize("which,value", [(2, np.nan), (2, np.inf), (1, -np.inf)])
+def test_non_finite(cuda, which, value):
+    def change(maps):
+        maps[which][7, 10, 3] = value
+    check(*run(20, 70, 60.0, 41, change))
