@@ -12,11 +12,10 @@
 //   z, r*h = gates of conv5x5(h, [W_z; W_r] over h) + cf
 //   h    = (1 - z) h + z tanh(conv5x5(r*h, W_q over h) + cf + b_q)
 //   prob, xy, angle = the three heads (conv3x3 -> ReLU -> conv1x1 -> ReLU -> conv1x1)
-//          on [h | uv], the 1x1 layers in the 3x3 layer's epilogue (the last
-//          iteration: all four heads)
+//          on [h | uv], the 1x1 layers in the 3x3 layer's epilogue
 //   pred = angmf_propagate(pred, prob, xy, angle) on logits  bvml_dsine_angmf_propagate_f32
-// and, in the last iteration only, the up-mask head and the convex upsample +
-// normalise with its bias (the reference computes an up-sampled map every
+// and, after the last iteration only, the up-mask head with the convex upsample +
+// normalise and the crop as its epilogue (the reference computes an up-sampled map every
 // iteration but returns the last one only, :276-283, :289-293, so the others
 // are dead work).  The convolutions add their bias once after their sum, in
 // the reference's rounding.
@@ -664,16 +663,12 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     const int out_h = a.out_h, out_w = a.out_w;
     float* out = a.out;
     float* coarse = a.coarse;
-    const size_t hw = (size_t)h8 * w8, b = sizeof(float);
-    const long long fh = (long long)kUp * h8, fw = (long long)kUp * w8;
+    const size_t hw = (size_t)h8 * w8;
     const hipStream_t strm = static_cast<hipStream_t>(stream);
     int st;
     // the grid-scaled intrinsics (src/dsine_refine.cpp:232-237)
     const double sw = (double)w8 / a.orig_w, sh = (double)h8 / a.orig_h;
     const double fu = a.fx * sw, cu = (a.cx + 0.5) * sw, fv = a.fy * sh, cv = (a.cy + 0.5) * sh;
-    auto copy = [&](float* dst, const float* src, size_t planes) {
-        return hipMemcpyAsync(dst, src, planes * hw * b, hipMemcpyDeviceToDevice, strm);
-    };
     // a kernel library status, with its message
     auto ck = [](int status, const char* what) {
         return status == BVML_DSINE_OK
@@ -683,7 +678,6 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     auto hip = [](hipError_t e, const char* what) {
         return e == hipSuccess ? BVML_DSINE_OK : hip_fail(e, what);
     };
-    hipError_t e;
     const Kernels* kern = kernels();
     if (!kern) return fail(BVML_DSINE_EUNSUP, "forward: built without the device kernels");
     // the camera's maps, pred = RayReLU(decoder.normal, ray_8) (:240-242), the
@@ -716,59 +710,51 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     update.xs = m.rs; update.x32 = m.rs; update.wp = r->w_q; update.cout = update.wcout = kHidden;
     update.s0 = m.cf + (size_t)2 * kHidden * hw; update.b0 = r->b_q; update.hf = m.hf;
     update.z = m.z; update.out = m.hf; update.outs = m.hs;
-    // the heads (:119-127, :257-267, :276): in the first four iterations the
-    // three the propagate reads, in the last all four; the up-mask head's last
-    // bias is the upsample's
+    // the heads the propagate reads (:119-127, :257-267)
     ConvArgs heads = base;
     heads.xs = m.hs; heads.x32 = m.hf; heads.tail = pa.th; heads.wp = r->w_h0;
-    heads.wcout = kHeads * kMid;
+    heads.wcout = kHeads * kMid; heads.cout = (kHeads - 1) * kMid;
     for (int h = 0; h < kHeads; ++h) {
         heads.w2[h] = r->w2[h];
         heads.w4[h] = r->w4[h];
         heads.hb0[h] = r->b_h[h][0];
         heads.hb2[h] = r->b_h[h][1];
-        heads.b4[h] = h < kHeads - 1 ? r->b_h[h][2] : nullptr;
-        heads.hout[h] = m.head[h];
+        heads.b4[h] = r->b_h[h][2];
+        heads.hout[h] = h < kHeads - 1 ? m.head[h] : nullptr;
         heads.nout[h] = kHeadOut[h];
     }
 
-    const bool direct = pad_t == 0 && pad_l == 0 && out_h == fh && out_w == fw;
-    int cur = 0;
+    // an iteration's heads and the next one's gates read the same hidden
+    // state: one launch
+    if ((st = hip(kern->conv(Conv::Gates, gates, strm), "gates convolution")) ||
+        (st = hip(kern->conv(Conv::Update, update, strm), "update convolution")))
+        return st;
+    const float* pred = m.pred[0];
     for (int it = 0; it < kIter; ++it) {
         const bool last = it == kIter - 1;
-        heads.cout = (last ? kHeads : kHeads - 1) * kMid;
-        if ((st = hip(kern->conv(Conv::Gates, gates, strm), "gates convolution")) ||
-            (st = hip(kern->conv(Conv::Update, update, strm), "update convolution")) ||
-            (st = hip(kern->conv(Conv::Heads, heads, strm), "heads convolution")))
+        if ((st = last ? hip(kern->conv(Conv::Heads, heads, strm), "heads convolution")
+                       : hip(kern->gates_heads(gates, heads, strm), "gates and heads")))
             return st;
-        // the propagate on the logits (:262-274)
-        if ((st = ck(bvml_dsine_angmf_propagate_f32(m.pred[cur], m.head[0], m.head[1],
-                                                    m.head[2], m.ray, fu, cu, fv, cv, 1, h8, w8,
-                                                    kPs, 0, m.pred[cur ^ 1], BVML_DSINE_LOGITS,
-                                                    stream), "angmf_propagate")))
+        // the propagate on the logits (:262-274), into the caller's coarse
+        // maps where they are asked for
+        float* dst = coarse ? coarse + (size_t)it * 3 * hw : m.pred[(it + 1) & 1];
+        if ((st = ck(bvml_dsine_angmf_propagate_f32(pred, m.head[0], m.head[1], m.head[2], m.ray,
+                                                    fu, cu, fv, cv, 1, h8, w8, kPs, 0, dst,
+                                                    BVML_DSINE_LOGITS, stream),
+                     "angmf_propagate")))
             return st;
-        cur ^= 1;
-        if (coarse && (e = copy(coarse + (size_t)it * 3 * hw, m.pred[cur], 3)) != hipSuccess)
-            return hip_fail(e, "hipMemcpyAsync");
-        if (!last) continue;
-        // up_pred_norm = normalize(convex_upsample(pred_norm, up_mask))  (:276-283)
-        float* dst = direct ? out : m.up;
-        if ((st = ck(bvml_dsine_convex_upsample_bias_f32(m.pred[cur], m.head[3], r->b_h[3][2], 1, 3,
-                                                         h8, w8, kUp, 1, kUpEps, dst, 0, stream),
-                     "convex_upsample")))
+        pred = dst;
+        if (!last && (st = hip(kern->conv(Conv::Update, update, strm), "update convolution")))
             return st;
     }
-    if (!direct) {
-        // the crop to the unpadded image (:289-293)
-        for (int c = 0; c < 3; ++c) {
-            const float* src = m.up + (size_t)c * fh * fw + (size_t)pad_t * fw + pad_l;
-            e = hipMemcpy2DAsync(out + (size_t)c * out_h * out_w, (size_t)out_w * b, src,
-                                 (size_t)fw * b, (size_t)out_w * b, (size_t)out_h,
-                                 hipMemcpyDeviceToDevice, strm);
-            if (e != hipSuccess) return hip_fail(e, "hipMemcpy2DAsync");
-        }
-    }
-    return BVML_DSINE_OK;
+    // up_pred_norm = normalize(convex_upsample(pred_norm, up_mask)) with the
+    // up-mask head (:276-283), cropped to the unpadded image (:289-293)
+    ConvArgs up = heads;
+    up.cout = kMid;
+    up.pred = pred; up.up = out; up.up_eps = kUpEps;
+    up.pad_t = pad_t; up.pad_l = pad_l; up.out_h = out_h; up.out_w = out_w;
+    up.up_vec4 = pad_l % 4 == 0 && out_w % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    return hip(kern->conv(Conv::Up, up, strm), "up-mask head and upsample");
 }
 
 int bvml_refine::refiner_device(const bvml_dsine_refiner* r) { return r->device; }

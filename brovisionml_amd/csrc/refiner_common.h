@@ -76,14 +76,13 @@ const std::vector<std::vector<float>>& host_weights(const bvml_dsine_refiner* r)
 // propagate buffers, the ray map, the full-resolution result before the crop,
 // the scales.
 struct Maps {
-    float *hf, *hs, *rs, *fs, *z, *cf, *uv, *th, *tf, *head[kHeads], *pred[2], *ray, *up, *info;
+    float *hf, *hs, *rs, *fs, *z, *cf, *uv, *th, *tf, *head[kHeads - 1], *pred[2], *ray, *info;
 };
 
-// The planes of each map in Maps order (up: 3 * kUp^2 planes), info apart;
+// The planes of each map in Maps order, info apart;
 // each map starts on a 64-float boundary.
 constexpr int kMapPlanes[] = {kHidden, kHidden, kHidden, kFeature, kHidden, 3 * kHidden,
-                              2, 2, 2, kHeadOut[0], kHeadOut[1], kHeadOut[2], kHeadOut[3],
-                              3, 3, 3, 3 * kUp * kUp};
+                              2, 2, 2, kHeadOut[0], kHeadOut[1], kHeadOut[2], 3, 3, 3};
 constexpr size_t kInfoFloats = 64 + 2 * 256;
 constexpr size_t maps_floats(size_t hw) {
     size_t total = kInfoFloats;
@@ -94,7 +93,7 @@ inline Maps maps_at(float* base, size_t hw) {
     Maps m{};
     float** order[] = {&m.hf,      &m.hs,      &m.rs,      &m.fs,      &m.z,       &m.cf,
                        &m.uv,      &m.th,      &m.tf,      &m.head[0], &m.head[1], &m.head[2],
-                       &m.head[3], &m.pred[0], &m.pred[1], &m.ray,     &m.up};
+                       &m.pred[0], &m.pred[1], &m.ray};
     static_assert(sizeof(order) / sizeof(order[0]) == sizeof(kMapPlanes) / sizeof(kMapPlanes[0]),
                   "one plane count per map");
     size_t at = 0;

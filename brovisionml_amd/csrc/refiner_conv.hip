@@ -28,6 +28,7 @@
 
 #include "angmf_ref.h"
 #include "refiner_kernels.h"
+#include "upsample_px.h"
 
 namespace {
 
@@ -35,15 +36,21 @@ using namespace bvml_refine;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTW = 16;  // tile width: one MFMA column block per tile row
 
-constexpr int kMaxOuts = 576;  // a head's outputs
+enum Epi : int { kPlain = 0, kGates = 1, kUpdate = 2, kHeads = 3, kUp = 4 };
 
-enum Epi : int { kPlain = 0, kGates = 1, kUpdate = 2, kHeads = 3 };
+// A head's small operands in LDS, in words: the three layers' exponents and
+// biases, [e0 64][b0 64][e2 64][b2 64][e4 outs][b4 outs], outs rounded up to
+// 16; the heads' outputs are at most 64, the up-mask head's 9 taps x 64.
+constexpr int kSubs = 64, kUpOuts = 9 * kSubs;
+constexpr int head_outs(int epi) { return epi == kUp ? kUpOuts : 64; }
+constexpr int head_words(int epi) { return 256 + 2 * head_outs(epi); }
 
 struct KArgs {
     ConvArgs c;
@@ -110,6 +117,9 @@ struct Shape {
     static constexpr int K = K_, MB = MB_, NB = NB_, WM = WM_, WN = WN_, KS = KS_, AD = AD_,
                          EPI = EPI_;
     static constexpr bool TAIL = TAIL_;
+    // registers for two waves on a SIMD, or (the up-mask head, with 9 blocks of
+    // weights resident) one: two spilled 430 bytes a lane
+    static constexpr int kWavesPerSimd = EPI == kUp ? 1 : 2;
     static constexpr int kWaves = WM * WN * KS, kThreads = 64 * kWaves;
     static constexpr int TH = NB * WN;
     static constexpr int HR = TH + K - 1, HC = kTW + K - 1, HS = HR * HC;
@@ -121,26 +131,29 @@ struct Shape {
     static constexpr int kTailBytes = TAIL ? 2 * kTailPx * 4 : 0;
     // the groups' partial sums, all but each group's own columns
     static constexpr int kXchBytes = KS > 1 ? WM * WN * (KS - 1) * MB * NB * 1024 : 0;
-    // the heads' operands and exponents
-    static constexpr int kHeadBytes = EPI == kHeads ? TH * 4416 + 64 + 8 * kMaxOuts : 0;
+    // the up-mask head's activations, their exponents, each row's flag
+    static constexpr int kFragBytes = EPI == kUp ? TH * (4096 + 64 + 16) : 0;
     static constexpr int kMainBytes = kHaloBytes + kTailBytes;
-    static constexpr int kLdsBytes = kMainBytes > kXchBytes
-                                         ? (kMainBytes > kHeadBytes ? kMainBytes : kHeadBytes)
-                                         : (kXchBytes > kHeadBytes ? kXchBytes : kHeadBytes);
+    static constexpr int kShared1 = kMainBytes > kXchBytes ? kMainBytes : kXchBytes;
+    static constexpr int kParamAt = ((kShared1 > kFragBytes ? kShared1 : kFragBytes) + 15) / 16 * 16;
+    static constexpr int kParamBytes = EPI >= kHeads ? WM * head_words(EPI) * 4 : 0;
+    // the up-mask head's normals, with a border of one pixel
+    static constexpr int kPredAt = kParamAt + kParamBytes;
+    static constexpr int kPredBytes = EPI == kUp ? (TH + 2) * (kTW + 2) * 16 : 0;
+    static constexpr int kLdsBytes = kPredAt + kPredBytes;
     static constexpr int NC = NB >= KS ? NB / KS : 1;  // columns (tile rows) a wave finishes
     static_assert(NB % KS == 0 || NB < KS, "whole columns per group");
-    static_assert(16 % kWaves == 0, "waves share a halo's 16 planes evenly");
     static_assert(AD % 2 == 0, "B operands alternate between two slots");
 };
 
+// Workgroup bx of nbx of one convolution.
 template <class S>
-__global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
+__device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char* lds) {
     constexpr int K = S::K, P = K / 2, TAPS = K * K, MAIN = 2 * TAPS;
     constexpr bool TAIL = S::TAIL;
     constexpr int STEPS = split_steps(K, TAIL);
     constexpr int MB = S::MB, NB = S::NB, WM = S::WM, WN = S::WN, KS = S::KS, AD = S::AD;
     constexpr int HC = S::HC, HS = S::HS, HSP = S::HSP, NC = S::NC, EPI = S::EPI;
-    __shared__ __align__(16) char lds[S::kLdsBytes];
 
     const ConvArgs& c = a.c;
     const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -150,11 +163,11 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
     // each XCD takes a contiguous run of (tile, channel group) pairs
     // (workgroups go to the 8 XCDs in turn), so neighbouring tiles share
     // their halo lines in one L2
-    const int nbx = (int)gridDim.x, bx = (int)blockIdx.x, xcd = bx & 7;
+    const int xcd = bx & 7;
     const int id = xcd * (nbx >> 3) + (xcd < (nbx & 7) ? xcd : (nbx & 7)) + (bx >> 3);
     const int tile = id / a.mgroups, mg = id - tile * a.mgroups;
     const int tx0 = (tile % a.tiles_x) * kTW, ty0 = (tile / a.tiles_x) * S::TH;
-    const int mb0 = mg * (MB * WM) + MB * wm;  // the wave's first M-block
+    const int mb0 = (EPI == kUp ? 12 : mg * (MB * WM)) + MB * wm;  // the wave's first M-block
     const int H = c.H, W = c.W;
     const size_t HW = a.HW;
 
@@ -166,8 +179,6 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
     const int* const wexp = reinterpret_cast<const int*>(c.wp);
     const uint32_t whead = split_head_words(a.wblocks);
     const Info* const info = reinterpret_cast<const Info*>(c.info);
-    const int xn = info->n[c.which];
-    const bool exact = info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
 
     const __amdgpu_buffer_rsrc_t wr = rsrc_of(c.wp + whead, (uint32_t)a.wblocks * STEPS * 2048u);
     const uint32_t lane16 = 16u * (uint32_t)lane;
@@ -181,61 +192,147 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
         }
     };
 
+    constexpr bool HEAD = EPI == kHeads || EPI == kUp;
+    constexpr int OUTS = head_outs(EPI);
+
+    // lane (g, col), register r of a block's sums is output channel
+    // 16 (mb0 + m) + 4 g + r (in the packed order) at pixel (row(j), tx0 + col)
+    const int x = tx0 + col;
+    auto row_of = [&](int j) { return ty0 + wn * NB + j * KS + ks; };
+    // channels 16 q + 4 g .. + 3 of a pixel, in c4
+    auto c4_at = [&](int q, uint32_t px) { return ((size_t)(4 * q + g) * HW + px) * 4; };
+    // what the gates' and the update's epilogues read, fetched before the sums
+    // where the reduction is split (few rows a wave, small grids), else after
+    constexpr bool EARLY = KS > 1 && (EPI == kGates || EPI == kUpdate);
+    constexpr int NE = EPI == kGates ? MB / 2 : EPI == kUpdate ? MB : 1;
+    v4f ep[3][NC][NE], eb[2][NE];
+    auto epilogue_loads = [&]() {
+        const int xc = x < W ? x : W - 1, q0 = EPI == kGates ? mb0 / 2 : mb0;
+#pragma unroll
+        for (int p = 0; p < NE; ++p) {
+            eb[0][p] = *reinterpret_cast<const v4f*>(c.b0 + 16 * (q0 + p) + 4 * g);
+            if (EPI == kGates)
+                eb[1][p] = *reinterpret_cast<const v4f*>(c.b1 + 16 * (q0 + p) + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int y = row_of(j) < H ? row_of(j) : H - 1;
+                const uint32_t px = (uint32_t)(y * W + xc);
+                const size_t at = c4_at(q0 + p, px);
+                if (EPI == kGates) {
+                    ep[0][j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p, px));
+                    ep[1][j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p + 1, px));
+                } else {
+                    ep[0][j][p] = *reinterpret_cast<const v4f*>(c.s0 + at);
+                    ep[1][j][p] = *reinterpret_cast<const v4f*>(c.z + at);
+                }
+                ep[2][j][p] = *reinterpret_cast<const v4f*>(c.hf + at);
+            }
+        }
+    };
+
     v4f acc[MB][NB];
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    if (!exact) {
-        // the halo to LDS with direct-to-LDS loads, 16 bytes a lane: each
-        // wave takes 16 / kWaves of the 16 planes (hi, lo x channel group)
-        const char* const xs = static_cast<const char*>(c.xs);
-        constexpr int PPW = 16 / S::kWaves;
+    // Everything the sums start from goes out before anything is waited for:
+    // one memory latency, where a grid is too small to hide several (whatever
+    // the scales turn out to be: the split map is allocated, if not written).
+    // the halo to LDS with direct-to-LDS loads, 16 bytes a lane: the waves
+    // share the 16 planes (hi, lo x channel group)
+    const char* const xs = static_cast<const char*>(c.xs);
+    constexpr int PPW = (16 + S::kWaves - 1) / S::kWaves;
+    const int pl0 = wave * PPW, pl1 = pl0 + PPW < 16 ? pl0 + PPW : 16;
 #pragma unroll
-        for (int ch = 0; ch < (HS + 63) / 64; ++ch) {
-            const int px = ch * 64 + lane;
-            const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
-            if (px < HS) {
-                if (y >= 0 && y < H && x >= 0 && x < W) {
-                    const char* src = xs + ((size_t)(wave * PPW) * HW + (uint32_t)(y * W + x)) * 16;
+    for (int ch = 0; ch < (HS + 63) / 64; ++ch) {
+        const int px = ch * 64 + lane;
+        const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
+        if (px < HS) {
+            if (y >= 0 && y < H && x >= 0 && x < W) {
+                const char* src = xs + ((size_t)pl0 * HW + (uint32_t)(y * W + x)) * 16;
 #pragma unroll
-                    for (int p = 0; p < PPW; ++p)
-                        __builtin_amdgcn_global_load_lds(
-                            static_cast<const void*>(src + (size_t)p * HW * 16),
-                            reinterpret_cast<__attribute__((address_space(3))) void*>(
-                                reinterpret_cast<uintptr_t>(
-                                    lds + ((wave * PPW + p) * HSP + ch * 64) * 16)),
-                            16, 0, 0);
-                } else {
+                for (int p = 0; p < PPW; ++p)
+                    if (16 % S::kWaves == 0 || pl0 + p < pl1) __builtin_amdgcn_global_load_lds(
+                        static_cast<const void*>(src + (size_t)p * HW * 16),
+                        reinterpret_cast<__attribute__((address_space(3))) void*>(
+                            reinterpret_cast<uintptr_t>(
+                                lds + ((pl0 + p) * HSP + ch * 64) * 16)),
+                        16, 0, 0);
+            } else {
 #pragma unroll
-                    for (int p = 0; p < PPW; ++p)
-                        *reinterpret_cast<v4u*>(lds + ((wave * PPW + p) * HSP + px) * 16) =
+                for (int p = 0; p < PPW; ++p)
+                    if (16 % S::kWaves == 0 || pl0 + p < pl1)
+                        *reinterpret_cast<v4u*>(lds + ((pl0 + p) * HSP + px) * 16) =
                             v4u{0, 0, 0, 0};
-                }
             }
         }
-        // the first steps' weights, in flight beside the halo
+    }
+    // the first steps' weights, in flight beside the halo
 #pragma unroll
-        for (int u = 0; u < AD; ++u) a_load(st0 + u < st1 ? st0 + u : st1 - 1, u);
-        uint32_t* const tl = reinterpret_cast<uint32_t*>(lds + S::kHaloBytes);
-        if constexpr (TAIL) {
+    for (int u = 0; u < AD; ++u) a_load(st0 + u < st1 ? st0 + u : st1 - 1, u);
+    uint32_t* const tl = reinterpret_cast<uint32_t*>(lds + S::kHaloBytes);
+    if constexpr (TAIL) {
 #pragma unroll
-            for (int i = 0; i < (S::kTailPx + S::kThreads - 1) / S::kThreads; ++i) {
-                const int px = tid + i * S::kThreads;
-                const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
-                const bool in = px < HS && y >= 0 && y < H && x >= 0 && x < W;
-                const uint32_t at = in ? (uint32_t)(y * W + x) : 0u;
-                const uint32_t hi = c.tail[at], lo = c.tail[HW + at];
-                if (px < S::kTailPx) {
-                    tl[px] = in ? hi : 0u;
-                    tl[S::kTailPx + px] = in ? lo : 0u;
-                }
+        for (int i = 0; i < (S::kTailPx + S::kThreads - 1) / S::kThreads; ++i) {
+            const int px = tid + i * S::kThreads;
+            const int y = ty0 + px / HC - P, x = tx0 + px % HC - P;
+            const bool in = px < HS && y >= 0 && y < H && x >= 0 && x < W;
+            const uint32_t at = in ? (uint32_t)(y * W + x) : 0u;
+            const uint32_t hi = c.tail[at], lo = c.tail[HW + at];
+            if (px < S::kTailPx) {
+                tl[px] = in ? hi : 0u;
+                tl[S::kTailPx + px] = in ? lo : 0u;
             }
         }
-        __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
-        __syncthreads();
+    }
+    // the heads' small operands, for the layers after the sums
+    if constexpr (HEAD) {
+        static_assert(!HEAD || MB == 4, "one head per wave");
+        for (int h = 0; h < WM; ++h) {
+            const int hd = EPI == kUp ? 3 : mg * WM + h;
+            const int nout = c.nout[hd];
+            const int* const e2 = reinterpret_cast<const int*>(c.w2[hd]);
+            const int* const e4 = reinterpret_cast<const int*>(c.w4[hd]);
+            int* const pe = reinterpret_cast<int*>(lds + S::kParamAt) + h * head_words(EPI);
+            float* const pb = reinterpret_cast<float*>(pe);
+            for (int i = tid; i < 64; i += S::kThreads) {
+                pe[i] = wexp[64 * hd + i];
+                pb[64 + i] = c.hb0[hd][i];
+                pe[128 + i] = e2[i];
+                pb[192 + i] = c.hb2[hd][i];
+            }
+            for (int i = tid; i < OUTS; i += S::kThreads) {
+                pe[256 + i] = i < (nout + 15) / 16 * 16 ? e4[i] : 0;
+                pb[256 + OUTS + i] = i < nout ? c.b4[hd][i] : 0.0f;
+            }
+        }
+    }
+    if constexpr (EPI == kUp) {
+        // each pixel's normal and its length (bvml::load_taps's)
+        for (int i = tid; i < (S::TH + 2) * (kTW + 2); i += S::kThreads) {
+            int y = ty0 + i / (kTW + 2) - 1, x = tx0 + i % (kTW + 2) - 1;
+            y = y < 0 ? 0 : y < H ? y : H - 1;
+            x = x < 0 ? 0 : x < W ? x : W - 1;
+            v4f v;
+            float s2 = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                v[k] = c.pred[k * HW + (uint32_t)(y * W + x)];
+                s2 = fmaf(v[k], v[k], s2);
+            }
+            v[3] = sqrtf(s2);
+            reinterpret_cast<v4f*>(lds + S::kPredAt)[i] = v;
+        }
+    }
 
+    if constexpr (EARLY) epilogue_loads();
+    const int xn = info->n[c.which];
+    const bool exact = info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
+    __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
+    __syncthreads();
+
+    if (!exact) {
         const char* const hb = lds + (g * HSP + wn * NB * HC + col) * 16;
         h8 bw[2][NB][2];
         auto b_load = [&](int st, int slot) {
@@ -336,6 +433,23 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
         }
     }
 
+    // the heads' second layer's weights, in flight through what follows
+    constexpr uint32_t kHead64 = split1x1_head_words(64);
+    h8 w2v[HEAD ? 4 : 1][2][2];
+    auto w_load = [&](__amdgpu_buffer_rsrc_t rr, int ob, h8 (&w)[2][2]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            w[q][0] = ld16(rr, lane16, (uint32_t)(ob * 2 + q) * 2048u);
+            w[q][1] = ld16(rr, lane16 + 1024u, (uint32_t)(ob * 2 + q) * 2048u);
+        }
+    };
+    const int hd = EPI == kUp ? 3 : HEAD ? mg * WM + wm : 0;
+    if constexpr (HEAD) {
+        const __amdgpu_buffer_rsrc_t r2 = rsrc_of(c.w2[hd] + kHead64, 4 * 2 * 2048u);
+#pragma unroll
+        for (int mo = 0; mo < 4; ++mo) w_load(r2, mo, w2v[mo]);
+    }
+
     // the groups' partial sums meet: group ks finishes columns n = ks, ks + KS, ...
     v4f own[MB][NC];
     if constexpr (KS > 1) {
@@ -351,7 +465,7 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
                 for (int m = 0; m < MB; ++m) xch[((n * MB + m) * (KS - 1) + k) * 64] = acc[m][n];
             }
         __syncthreads();
-        if (EPI != kHeads && ks >= NB) return;
+        if (EPI != kUp && ks >= NB) return;
 #pragma unroll
         for (int n = 0; n < NB; ++n)
             if (n % KS == ks) {
@@ -370,12 +484,8 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
             for (int n = 0; n < NB; ++n) own[m][n] = acc[m][n];
     }
 
-    // epilogue: lane (g, col), register r of own[m][j] is output channel
-    // 16 (mb0 + m) + 4 g + r (in the packed order) at pixel (row(j), tx0 + col)
-    const int x = tx0 + col;
-    auto row_of = [&](int j) { return ty0 + wn * NB + j * KS + ks; };
     // the scales come off
-    if (!exact) {
+    if (!HEAD && !exact) {
 #pragma unroll
         for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -385,8 +495,7 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
                 for (int j = 0; j < NC; ++j) own[m][j][r] = ldexpf(own[m][j][r], e);
             }
     }
-    // channels 16 q + 4 g .. + 3 of a pixel, in c4 and in a split map
-    auto c4_at = [&](int q, uint32_t px) { return ((size_t)(4 * q + g) * HW + px) * 4; };
+    // the same channels to a split map
     auto store_split = [&](void* base, int q, uint32_t px, const v4f& v) {
         float s[4];
 #pragma unroll
@@ -398,289 +507,335 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
         *reinterpret_cast<h4*>(p + 8 * HW * 16) = lo;
     };
 
-    if constexpr (EPI == kHeads) {
-        // The rest of head mg on the matrix cores, the workgroup's waves
-        // sharing the tile's activations through LDS as operands:
+    if constexpr (HEAD) {
+        // The rest of a head on the matrix cores, in the registers of the wave
+        // that has its sums:
         //   a = relu(s + b0);  t = relu(W2 a + b2);  out = W4 t + b4.
         // A 1x1 layer's reduction step of 32 channels takes M-blocks 2q and
         // 2q + 1: lane (g, col) holds their channels 16 m + 4 g + r, which is
         // its B operand, the weights being packed in that channel order.  Each
-        // pixel's channels are scaled to their largest and split.  (Each wave
-        // running both layers for its own columns took 107 us for the three
-        // heads at 256 x 256 and 405 us for all four: every wave streamed
-        // every weight, one load's latency per 16 outputs.)
-        static_assert(EPI != kHeads || (MB == 4 && WM == 1), "one head per wave");
-        static_assert(EPI != kHeads || (S::kWaves % 4 == 0 && S::TH % (S::kWaves / 4) == 0 &&
-                                        S::TH % 2 == 0), "the waves share the layers");
-        constexpr int TH = S::TH;
-        // LDS: the operands [q 0, 1][hi, lo][row][lane] 16 bytes (or the fp32
-        // activations [m][row][lane], where one is infinite or NaN), each
-        // pixel's exponent in the first layer, its largest t per M-block, the
-        // waves' largest, the last layer's exponents and biases
-        char* const frag = lds;
-        int* const e1 = reinterpret_cast<int*>(lds + TH * 4096);
-        uint32_t* const pm = reinterpret_cast<uint32_t*>(lds + TH * 4096 + TH * 64);
-        uint32_t* const red = reinterpret_cast<uint32_t*>(lds + TH * 4096 + TH * 320);
-        int* const e4s = reinterpret_cast<int*>(lds + TH * 4416 + 64);
-        float* const b4s = reinterpret_cast<float*>(e4s + kMaxOuts);
-        const int hd = mg;
-        const float* w2 = c.w2[hd];
-        const float* w4 = c.w4[hd];
-        const float* b4 = c.b4[hd];
-        float* out = c.hout[hd];
+        // pixel's channels are scaled to their largest and split; a row with an
+        // infinity or a NaN (or weights with one) takes fp32 products.  (The
+        // waves sharing the layers through LDS, six barriers a workgroup, took
+        // 99 us for the three heads at 256 x 256 against 61; two waves a SIMD
+        // matter more than what a third shape would save: 85 us where the
+        // registers allowed one.)
+        const int* const pe = reinterpret_cast<const int*>(lds + S::kParamAt) + wm * head_words(EPI);
+        const float* const pb = reinterpret_cast<const float*>(pe);
+        auto e_at = [&](int at) { return *reinterpret_cast<const v4i*>(pe + at + 4 * g); };
+        auto b_of = [&](int at) { return *reinterpret_cast<const v4f*>(pb + at + 4 * g); };
+        const float* const w2 = c.w2[hd];
+        const float* const w4 = c.w4[hd];
         const int nout = c.nout[hd], nob = (nout + 15) / 16;
-        constexpr uint32_t kHead64 = split1x1_head_words(64);
         const uint32_t head4 = split1x1_head_words(nout);
-        const __amdgpu_buffer_rsrc_t r2 = rsrc_of(w2 + kHead64, 4 * 2 * 2048u);
         const __amdgpu_buffer_rsrc_t r4 = rsrc_of(w4 + head4, (uint32_t)nob * 2 * 2048u);
-        const int* e2 = reinterpret_cast<const int*>(w2);
-        const int* e4 = reinterpret_cast<const int*>(w4);
-        const bool ok2 = e2[64] != 0, ok4 = e4[16 * nob] != 0;
-        auto w_load = [&](__amdgpu_buffer_rsrc_t rr, int ob, h8 (&w)[2][2]) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                w[q][0] = ld16(rr, lane16, (uint32_t)(ob * 2 + q) * 2048u);
-                w[q][1] = ld16(rr, lane16 + 1024u, (uint32_t)(ob * 2 + q) * 2048u);
-            }
-        };
-        auto frag_at = [&](int q, int hl, int row) {
-            return reinterpret_cast<h8*>(frag + (((q * 2 + hl) * TH + row) * 64 + lane) * 16);
-        };
-        auto act_at = [&](int m, int row) {
-            return reinterpret_cast<v4f*>(frag + ((m * TH + row) * 64 + lane) * 16);
-        };
-        // 16 outputs for one row of pixels, split and fp32
-        auto split16 = [&](const h8 (&w)[2][2], const h8 (&b)[2][2], v4f o) {
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    o = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[q][p == 0 ? 1 : 0],
-                                                               b[q][p == 1 ? 1 : 0], o, 0, 0, 0);
-            return o;
-        };
-        auto exact16 = [&](const float* w32, int ob, int row) {
+        const bool ok2 = reinterpret_cast<const int*>(w2)[64] != 0;
+        const bool ok4 = reinterpret_cast<const int*>(w4)[16 * nob] != 0;
+        auto exact16 = [&](const float* w32, int ob, const v4f (&v)[4]) {
             v4f o = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            for (int m = 0; m < 4; ++m) {
-                const v4f v = *act_at(m, row);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     o = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        w32[((size_t)ob * 16 + 4 * m + r) * 64 + lane], v[r], o, 0, 0, 0);
-            }
+                        w32[((size_t)ob * 16 + 4 * m + r) * 64 + lane], v[m][r], o, 0, 0, 0);
             return o;
         };
-
-        h8 wa[2][2];
-        const int mo = wave & 3;  // the wave's M-block of t
-        w_load(r2, mo, wa);
-        // a of the wave's own columns, and their pixels' largest
-        uint32_t mx[NC], top = 0;
-        if (ks < NB) {
-            v4f b0v[4];
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-                b0v[m] = *reinterpret_cast<const v4f*>(c.hb0[hd] + 16 * m + 4 * g);
-#pragma unroll
-            for (int j = 0; j < NC; ++j) {
-                mx[j] = 0;
-#pragma unroll
-                for (int m = 0; m < 4; ++m)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        own[m][j][r] = relu(own[m][j][r] + b0v[m][r]);
-                        mx[j] = umax(mx[j], absbits(own[m][j][r]));
-                    }
-                mx[j] = umax(mx[j], (uint32_t)__shfl_xor((int)mx[j], 16));
-                mx[j] = umax(mx[j], (uint32_t)__shfl_xor((int)mx[j], 32));
-                top = umax(top, mx[j]);
-            }
-        }
-        __syncthreads();  // the partial sums are read
-        for (int i = tid; i < 16 * nob; i += S::kThreads) {
-            e4s[i] = e4[i];
-            b4s[i] = b4 && i < nout ? b4[i] : 0.0f;
-        }
-        top = wave_max(top);
-        if (lane == 0) red[wave] = top;
-        __syncthreads();
-        bool ok = ok2;
-#pragma unroll
-        for (int w = 0; w < S::kWaves; ++w) ok = ok && red[w] < kInfBits;
-        if (ks < NB) {
-#pragma unroll
-            for (int j = 0; j < NC; ++j) {
-                const int row = wn * NB + j * KS + ks;
-                if (ok) {
-                    const int n = scale_exp(mx[j]);
-                    const float sc = pow2(n);
-                    if (g == 0) e1[row * 16 + col] = -n;
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        float s[8];
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) s[i] = own[2 * q + (i >> 2)][j][i & 3] * sc;
-                        h8 hi, lo;
-                        split_to(s, hi, lo);
-                        *frag_at(q, 0, row) = hi;
-                        *frag_at(q, 1, row) = lo;
-                    }
-                } else {
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) *act_at(m, row) = own[m][j];
-                }
-            }
-        }
-        __syncthreads();
-        // t = relu(W2 a + b2): M-block mo of the rows of the wave's share
-        constexpr int R1 = TH / (S::kWaves / 4);
-        const int row1 = (wave >> 2) * R1;
-        v4f t[R1];
-        uint32_t tm[R1];
-        {
-            const v4f b2v = *reinterpret_cast<const v4f*>(c.hb2[hd] + 16 * mo + 4 * g);
-            int ew[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ew[r] = e2[16 * mo + 4 * g + r];
-            top = 0;
-#pragma unroll
-            for (int j = 0; j < R1; ++j) {
-                const int row = row1 + j;
-                v4f o;
-                if (ok) {
-                    h8 b[2][2];
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        b[q][0] = *frag_at(q, 0, row);
-                        b[q][1] = *frag_at(q, 1, row);
-                    }
-                    o = split16(wa, b, v4f{0.0f, 0.0f, 0.0f, 0.0f});
-                    const int ex = e1[row * 16 + col];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) o[r] = ldexpf(o[r], ew[r] + ex);
-                } else {
-                    o = exact16(w2 + kHead64 + 4096, mo, row);
-                }
-                tm[j] = 0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    t[j][r] = relu(o[r] + b2v[r]);
-                    tm[j] = umax(tm[j], absbits(t[j][r]));
-                }
-                tm[j] = umax(tm[j], (uint32_t)__shfl_xor((int)tm[j], 16));
-                tm[j] = umax(tm[j], (uint32_t)__shfl_xor((int)tm[j], 32));
-                if (g == 0) pm[(mo * TH + row) * 16 + col] = tm[j];
-                top = umax(top, tm[j]);
-            }
-        }
-        top = wave_max(top);
-        __syncthreads();  // a is read
-        if (lane == 0) red[wave] = top;
-        // the last layer's first weights: block `wave / 2` and on, by kWaves / 2
-        constexpr int OBS = S::kWaves / 2;
-        const int ob0 = wave >> 1;
-        if (ok4) w_load(r4, ob0 < nob ? ob0 : nob - 1, wa);
-        __syncthreads();
-        ok = ok4;
-#pragma unroll
-        for (int w = 0; w < S::kWaves; ++w) ok = ok && red[w] < kInfBits;
-        auto px_exp = [&](int row) {
+        // a pixel's largest magnitude over its 64 channels
+        auto px_max = [&](const v4f (&v)[4]) {
             uint32_t m = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) m = umax(m, pm[(k * TH + row) * 16 + col]);
-            return scale_exp(m);
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) m = umax(m, absbits(v[k][r]));
+            m = umax(m, (uint32_t)__shfl_xor((int)m, 16));
+            return umax(m, (uint32_t)__shfl_xor((int)m, 32));
         };
+        auto operands = [&](const v4f (&v)[4], float sc, h8 (&b)[2][2]) {
 #pragma unroll
-        for (int j = 0; j < R1; ++j) {
-            const int row = row1 + j;
-            if (ok) {
-                const float sc = pow2(px_exp(row));
-                float s[4];
+            for (int q = 0; q < 2; ++q) {
+                float s[8];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) s[r] = t[j][r] * sc;
-                h4 hi, lo;
-                split_to(s, hi, lo);
-                reinterpret_cast<h4*>(frag_at(mo >> 1, 0, row))[mo & 1] = hi;
-                reinterpret_cast<h4*>(frag_at(mo >> 1, 1, row))[mo & 1] = lo;
-            } else {
-                *act_at(mo, row) = t[j];
+                for (int i = 0; i < 8; ++i) s[i] = v[2 * q + (i >> 2)][i & 3] * sc;
+                split_to(s, b[q][0], b[q][1]);
             }
-        }
-        __syncthreads();
-        // out = W4 t + b4: a wave takes one half of the rows and every OBS-th
-        // block of 16 outputs, its operands in registers
-        constexpr int R2 = TH / 2;
-        const int row2 = (wave & 1) * R2;
-        h8 b[R2][2][2];
-        int ex[R2];
-        if (ok) {
+        };
+        // t of the wave's rows as operands (or, where one is infinite or NaN,
+        // as fp32 values), its exponents, and the rows that are operands
+        v4u tb[NC][4];
+        int ex[NC];
+        uint32_t split_rows = 0;
+        h8 wa[2][2][2];
+        if constexpr (EPI == kHeads) w_load(r4, 0, wa[0]);
+        if (KS == 1 || ks < NB) {
 #pragma unroll
-            for (int j = 0; j < R2; ++j) {
-                ex[j] = -px_exp(row2 + j);
+            for (int j = 0; j < NC; ++j) {
+                v4f act[4], t[4];
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    b[j][q][0] = *frag_at(q, 0, row2 + j);
-                    b[j][q][1] = *frag_at(q, 1, row2 + j);
+                for (int m = 0; m < 4; ++m) {
+                    const v4i e = e_at(16 * m);
+                    const v4f b = b_of(64 + 16 * m);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = own[m][j][r];
+                        act[m][r] = relu((exact ? v : ldexpf(v, e[r] - xn)) + b[r]);
+                    }
+                }
+                const uint32_t am = px_max(act);
+                if (ok2 && __all(am < kInfBits)) {
+                    const int n = scale_exp(am);
+                    h8 b[2][2];
+                    operands(act, pow2(n), b);
+#pragma unroll
+                    for (int mo = 0; mo < 4; ++mo) t[mo] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+#pragma unroll
+                            for (int mo = 0; mo < 4; ++mo)
+                                t[mo] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    w2v[mo][q][p == 0 ? 1 : 0], b[q][p == 1 ? 1 : 0], t[mo], 0, 0,
+                                    0);
+#pragma unroll
+                    for (int mo = 0; mo < 4; ++mo) {
+                        const v4i e = e_at(128 + 16 * mo);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) t[mo][r] = ldexpf(t[mo][r], e[r] - n);
+                    }
+                } else {
+#pragma unroll
+                    for (int mo = 0; mo < 4; ++mo) t[mo] = exact16(w2 + kHead64 + 4096, mo, act);
+                }
+#pragma unroll
+                for (int mo = 0; mo < 4; ++mo) {
+                    const v4f b = b_of(192 + 16 * mo);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) t[mo][r] = relu(t[mo][r] + b[r]);
+                }
+                const uint32_t tm = px_max(t);
+                ex[j] = 0;
+                if (ok4 && __all(tm < kInfBits)) {
+                    const int n = scale_exp(tm);
+                    h8 b[2][2];
+                    operands(t, pow2(n), b);
+                    ex[j] = -n;
+                    split_rows |= 1u << j;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        tb[j][i] = __builtin_bit_cast(v4u, b[i >> 1][i & 1]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) tb[j][i] = __builtin_bit_cast(v4u, t[i]);
                 }
             }
         }
-        // (The loop's only loads are the weights, issued before the stores of
-        // the block before; the stores are buffer stores, dropped beyond the
-        // map by their offset, not by a branch, so that their count is known:
-        // loads and stores share one counter, and with the exponents and
-        // biases loaded here each block waited for the last one's stores, 458
-        // us for the four heads at 256 x 256.)
-        uint32_t at[R2];
+        auto exact_out = [&](int ob, const v4u (&b)[4]) {
+            v4f v[4];
 #pragma unroll
-        for (int j = 0; j < R2; ++j) {
-            const int y = ty0 + row2 + j;
-            at[j] = x < W && y < H ? 4u * (uint32_t)(4 * g * a.HW + y * W + x) : 0xf0000000u;
-        }
-        auto store16 = [&](int ob, const v4f (&o)[R2]) {
-            const int left = nout - 16 * ob;
-            const __amdgpu_buffer_rsrc_t ro =
-                rsrc_of(out + (size_t)16 * ob * HW, (uint32_t)(left < 16 ? left : 16) * a.HW * 4u);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float bias = b4s[16 * ob + 4 * g + r];
-#pragma unroll
-                for (int j = 0; j < R2; ++j)
-                    __builtin_amdgcn_raw_buffer_store_b32(
-                        __builtin_bit_cast(uint32_t, b4 ? o[j][r] + bias : o[j][r]), ro,
-                        (int)(at[j] + (uint32_t)r * 4u * a.HW), 0, 0);
-            }
+            for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(v4f, b[i]);
+            return exact16(w4 + head4 + (size_t)nob * 1024, ob, v);
         };
-        if (ok) {
-            auto block = [&](int ob) {
-                v4f o[R2];
+        if constexpr (EPI == kHeads) {
+            // (Buffer stores, dropped beyond the map and the head's planes by
+            // their offset, not by a branch.)
+            float* const out = c.hout[hd];
+            uint32_t at[NC];
 #pragma unroll
-                for (int j = 0; j < R2; ++j)
-                    o[j] = split16(wa, b[j], v4f{0.0f, 0.0f, 0.0f, 0.0f});
-                __builtin_amdgcn_sched_barrier(0);
-                w_load(r4, ob + OBS < nob ? ob + OBS : ob, wa);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < NC; ++j) {
+                const int y = row_of(j);
+                at[j] = x < W && y < H ? 4u * (uint32_t)(4 * g * a.HW + y * W + x) : 0xf0000000u;
+            }
+            auto store16 = [&](int ob, const v4f (&o)[NC]) {
+                const int left = nout - 16 * ob;
+                const __amdgpu_buffer_rsrc_t ro = rsrc_of(
+                    out + (size_t)16 * ob * HW, (uint32_t)(left < 16 ? left : 16) * a.HW * 4u);
+                const v4f b = b_of(256 + OUTS + 16 * ob);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int ew = e4s[16 * ob + 4 * g + r];
+                for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int j = 0; j < R2; ++j) o[j][r] = ldexpf(o[j][r], ew + ex[j]);
-                }
+                    for (int j = 0; j < NC; ++j)
+                        __builtin_amdgcn_raw_buffer_store_b32(
+                            __builtin_bit_cast(uint32_t, o[j][r] + b[r]), ro,
+                            (int)(at[j] + (uint32_t)r * 4u * a.HW), 0, 0);
+            };
+            auto block = [&](int ob, const h8 (&w)[2][2]) {
+                v4f o[NC];
+#pragma unroll
+                for (int j = 0; j < NC; ++j) o[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int j = 0; j < NC; ++j)
+                            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                w[q][p == 0 ? 1 : 0],
+                                __builtin_bit_cast(h8, tb[j][2 * q + (p == 1 ? 1 : 0)]), o[j], 0, 0,
+                                0);
+                const v4i e = e_at(256 + 16 * ob);
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[j][r] = ldexpf(o[j][r], e[r] + ex[j]);
                 store16(ob, o);
             };
-            // (the first block apart: at the loop's head the weights are then
-            // always followed by one block's stores, which their wait leaves
-            // in flight)
-            if (ob0 < nob) {
-                block(ob0);
-                for (int ob = ob0 + OBS; ob < nob; ob += OBS) block(ob);
+            if (split_rows == (1u << NC) - 1) {
+                for (int ob = 0; ob < nob; ob += 2) {
+                    w_load(r4, ob + 1 < nob ? ob + 1 : ob, wa[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    block(ob, wa[0]);
+                    if (ob + 1 >= nob) break;
+                    w_load(r4, ob + 2 < nob ? ob + 2 : ob, wa[0]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    block(ob + 1, wa[1]);
+                }
+            } else {
+                for (int ob = 0; ob < nob; ++ob) {
+                    v4f o[NC];
+                    w_load(r4, ob, wa[0]);
+#pragma unroll
+                    for (int j = 0; j < NC; ++j) {
+                        if (split_rows >> j & 1) {
+                            v4f v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                                for (int q = 0; q < 2; ++q)
+                                    v = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                        wa[0][q][p == 0 ? 1 : 0],
+                                        __builtin_bit_cast(h8, tb[j][2 * q + (p == 1 ? 1 : 0)]), v,
+                                        0, 0, 0);
+                            const v4i e = e_at(256 + 16 * ob);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) o[j][r] = ldexpf(v[r], e[r] + ex[j]);
+                        } else {
+                            o[j] = exact_out(ob, tb[j]);
+                        }
+                    }
+                    store16(ob, o);
+                }
             }
         } else {
-            for (int ob = ob0; ob < nob; ob += OBS) {
-                v4f o[R2];
+            // The up-mask head's last layer, the convex upsample of the normals
+            // by its 9 x 64 outputs and their normalise: wave sb takes
+            // sub-pixels 16 sb .. + 15 of every pixel of the tile, so a lane
+            // has all 9 taps of its 4 sub-pixels in registers and no mask is
+            // written.  Its weights, 9 blocks of 16 outputs, stay in registers
+            // over the rows; the activations come from the waves that have
+            // them through LDS.  256 x 256: 75 us against 97 for the head
+            // writing 151 MB of mask and 42 for the upsample reading them;
+            // about half is the upsample's vector arithmetic.
+            static_assert(EPI != kUp || S::kWaves == 4, "a quarter of the sub-pixels a wave");
+            h8 w9[9][2][2];
 #pragma unroll
-                for (int j = 0; j < R2; ++j)
-                    o[j] = exact16(w4 + head4 + (size_t)nob * 1024, ob, row2 + j);
-                store16(ob, o);
+            for (int n = 0; n < 9; ++n) w_load(r4, 4 * n + wave, w9[n]);
+            int* const exl = reinterpret_cast<int*>(lds + S::TH * 4096);
+            int* const rowok = reinterpret_cast<int*>(lds + S::TH * (4096 + 64));
+            __syncthreads();  // the halo or the partial sums are read
+            if (KS == 1 || ks < NB) {
+#pragma unroll
+                for (int j = 0; j < NC; ++j) {
+                    const int row = wn * NB + j * KS + ks;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        reinterpret_cast<v4u*>(lds)[(row * 4 + i) * 64 + lane] = tb[j][i];
+                    if (g == 0) exl[row * 16 + col] = ex[j];
+                    if (lane == 0) rowok[4 * row] = split_rows >> j & 1;
+                }
+            }
+            __syncthreads();
+            const double eps = c.up_eps;
+            const float eps_s = (float)(1.01 * eps);
+            const int sub0 = 16 * wave + 4 * g;  // the lane's first sub-pixel
+            const int oy0 = sub0 / 8 - c.pad_t, ox = 8 * x + sub0 % 8 - c.pad_l;
+            for (int row = 0; row < S::TH && ty0 + row < H; ++row) {
+                v4u b[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    b[i] = reinterpret_cast<const v4u*>(lds)[(row * 4 + i) * 64 + lane];
+                v4f m[9];
+                if (__builtin_amdgcn_readfirstlane(rowok[4 * row])) {
+                    const int xe = exl[row * 16 + col];
+#pragma unroll
+                    for (int n = 0; n < 9; ++n) m[n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+#pragma unroll
+                            for (int n = 0; n < 9; ++n)
+                                m[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    w9[n][q][p == 0 ? 1 : 0],
+                                    __builtin_bit_cast(h8, b[2 * q + (p == 1 ? 1 : 0)]), m[n], 0,
+                                    0, 0);
+#pragma unroll
+                    for (int n = 0; n < 9; ++n) {
+                        const v4i e = e_at(256 + kSubs * n + 16 * wave);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) m[n][r] = ldexpf(m[n][r], e[r] + xe);
+                    }
+                } else {
+#pragma unroll
+                    for (int n = 0; n < 9; ++n) m[n] = exact_out(4 * n + wave, b);
+                }
+                bvml::Taps<3> tp;
+                float q_sum = 0.0f;
+#pragma unroll
+                for (int n = 0; n < 9; ++n) {
+                    m[n] += b_of(256 + OUTS + kSubs * n + 16 * wave);
+                    const v4f v = reinterpret_cast<const v4f*>(
+                        lds + S::kPredAt)[(row + n / 3) * (kTW + 2) + col + n % 3];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) tp.v[k][n] = v[k];
+                    tp.nrm[n] = v[3];
+                    q_sum += v[3];
+                }
+                tp.flush = bvml::kFlushAbs * q_sum;
+                float o[3][4];
+                unsigned redo = 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float mr[9], res[3];
+#pragma unroll
+                    for (int n = 0; n < 9; ++n) mr[n] = m[n][r];
+                    const bool ok = bvml::fast_subpixel<3>(mr, tp, bvml::kNormalize, eps_s, res);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) o[k][r] = res[k];
+                    redo |= (ok ? 0u : 1u) << r;
+                }
+                while (redo) {
+                    const int r = __builtin_ctz(redo);
+                    redo &= redo - 1;
+                    float mr[9], res[3];
+#pragma unroll
+                    for (int n = 0; n < 9; ++n)
+                        mr[n] = r == 0 ? m[n][0] : r == 1 ? m[n][1] : r == 2 ? m[n][2] : m[n][3];
+                    bvml::exact_subpixel<3>(mr, tp, true, eps, res);
+#pragma unroll
+                    for (int rr = 0; rr < 4; ++rr)
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) o[k][rr] = r == rr ? res[k] : o[k][rr];
+                }
+                const int oy = 8 * (ty0 + row) + oy0;
+                if (x >= W || oy < 0 || oy >= c.out_h) continue;
+                float* dst = c.up + (size_t)oy * c.out_w;
+                const size_t plane = (size_t)c.out_h * c.out_w;
+                if (c.up_vec4) {
+                    // (all four columns are inside, or none)
+                    if (ox >= 0 && ox < c.out_w)
+#pragma unroll
+                        for (int k = 0; k < 3; ++k)
+                            __builtin_nontemporal_store(
+                                v4f{o[k][0], o[k][1], o[k][2], o[k][3]},
+                                reinterpret_cast<v4f*>(dst + k * plane + ox));
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (ox + r >= 0 && ox + r < c.out_w)
+#pragma unroll
+                            for (int k = 0; k < 3; ++k) dst[k * plane + ox + r] = o[k][r];
+                }
             }
         }
     } else if constexpr (EPI == kPlain) {
@@ -699,22 +854,9 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
         // (the compiler cannot know that they do not overlap)
         constexpr int MP = MB / 2;
         static_assert(EPI != kGates || MB % 2 == 0, "z and r blocks in pairs");
+        if constexpr (!EARLY) epilogue_loads();
         if (x >= W) return;
         const int q0 = mb0 / 2;
-        v4f sz[NC][MP], sr[NC][MP], hv[NC][MP], bz[MP], br[MP];
-#pragma unroll
-        for (int p = 0; p < MP; ++p) {
-            bz[p] = *reinterpret_cast<const v4f*>(c.b0 + 16 * (q0 + p) + 4 * g);
-            br[p] = *reinterpret_cast<const v4f*>(c.b1 + 16 * (q0 + p) + 4 * g);
-#pragma unroll
-            for (int j = 0; j < NC; ++j) {
-                const int y = row_of(j) < H ? row_of(j) : H - 1;
-                const uint32_t px = (uint32_t)(y * W + x);
-                sz[j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p, px));
-                sr[j][p] = *reinterpret_cast<const v4f*>(c.s0 + c4_at(mb0 + 2 * p + 1, px));
-                hv[j][p] = *reinterpret_cast<const v4f*>(c.hf + c4_at(q0 + p, px));
-            }
-        }
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             const int y = row_of(j);
@@ -725,8 +867,9 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
                 v4f zz, rh;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    zz[r] = sigmoid(own[2 * p][j][r] + sz[j][p][r] + bz[p][r]);
-                    rh[r] = sigmoid(own[2 * p + 1][j][r] + sr[j][p][r] + br[p][r]) * hv[j][p][r];
+                    zz[r] = sigmoid(own[2 * p][j][r] + ep[0][j][p][r] + eb[0][p][r]);
+                    rh[r] = sigmoid(own[2 * p + 1][j][r] + ep[1][j][p][r] + eb[1][p][r]) *
+                            ep[2][j][p][r];
                 }
                 *reinterpret_cast<v4f*>(c.z + c4_at(q0 + p, px)) = zz;
                 if (info->exact[0])
@@ -736,20 +879,8 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
             }
         }
     } else {
+        if constexpr (!EARLY) epilogue_loads();
         if (x >= W) return;
-        v4f bq[MB], sq[NC][MB], zv[NC][MB], hv[NC][MB];
-#pragma unroll
-        for (int m = 0; m < MB; ++m) {
-            bq[m] = *reinterpret_cast<const v4f*>(c.b0 + 16 * (mb0 + m) + 4 * g);
-#pragma unroll
-            for (int j = 0; j < NC; ++j) {
-                const int y = row_of(j) < H ? row_of(j) : H - 1;
-                const size_t at = c4_at(mb0 + m, (uint32_t)(y * W + x));
-                sq[j][m] = *reinterpret_cast<const v4f*>(c.s0 + at);
-                zv[j][m] = *reinterpret_cast<const v4f*>(c.z + at);
-                hv[j][m] = *reinterpret_cast<const v4f*>(c.hf + at);
-            }
-        }
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             const int y = row_of(j);
@@ -760,8 +891,8 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
                 v4f hn;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    hn[r] = gru_mix(zv[j][m][r], hv[j][m][r],
-                                    tanhf(own[m][j][r] + sq[j][m][r] + bq[m][r]));
+                    hn[r] = gru_mix(ep[1][j][m][r], ep[2][j][m][r],
+                                    tanhf(own[m][j][r] + ep[0][j][m][r] + eb[0][m][r]));
                 *reinterpret_cast<v4f*>(c.out + c4_at(mb0 + m, px)) = hn;
                 if (!info->exact[0]) store_split(c.outs, mb0 + m, px, hn);
             }
@@ -770,17 +901,52 @@ __global__ __launch_bounds__(S::kThreads) void conv_kernel(KArgs a) {
 }
 
 template <class S>
-hipError_t launch(const ConvArgs& c, hipStream_t stream) {
-    KArgs a{};
+__global__ __launch_bounds__(S::kThreads, S::kWavesPerSimd) void conv_kernel(KArgs a) {
+    __shared__ __align__(16) char lds[S::kLdsBytes];
+    conv_group<S>(a, (int)blockIdx.x, (int)gridDim.x, lds);
+}
+
+// Two convolutions that do not depend on each other: the first nb blocks do
+// b's, the others a's.
+template <class A, class B>
+__global__ __launch_bounds__(A::kThreads, 2) void pair_kernel(KArgs a, KArgs b, int nb) {
+    static_assert(A::kThreads == B::kThreads, "one block size");
+    __shared__ __align__(16) char lds[A::kLdsBytes > B::kLdsBytes ? A::kLdsBytes : B::kLdsBytes];
+    const int bx = (int)blockIdx.x;
+    if (bx < nb)
+        conv_group<B>(b, bx, nb, lds);
+    else
+        conv_group<A>(a, bx - nb, (int)gridDim.x - nb, lds);
+}
+
+// The launch's arguments and workgroups.
+template <class S>
+long long shape_args(const ConvArgs& c, KArgs& a) {
+    a = KArgs{};
     a.c = c;
     a.wblocks = c.wcout / 16;
     a.HW = (uint32_t)((size_t)c.H * c.W);
     a.tiles_x = (c.W + kTW - 1) / kTW;
     a.mgroups = c.cout / (16 * S::MB * S::WM);
-    const long long groups =
-        (long long)a.tiles_x * ((c.H + S::TH - 1) / S::TH) * a.mgroups;
+    return (long long)a.tiles_x * ((c.H + S::TH - 1) / S::TH) * a.mgroups;
+}
+
+template <class S>
+hipError_t launch(const ConvArgs& c, hipStream_t stream) {
+    KArgs a;
+    const long long groups = shape_args<S>(c, a);
     if (groups > INT_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL((conv_kernel<S>), dim3((unsigned)groups), dim3(S::kThreads), 0, stream, a);
+    return hipGetLastError();
+}
+
+template <class A, class B>
+hipError_t launch_pair(const ConvArgs& ca, const ConvArgs& cb, hipStream_t stream) {
+    KArgs a, b;
+    const long long na = shape_args<A>(ca, a), nb = shape_args<B>(cb, b);
+    if (na + nb > INT_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((pair_kernel<A, B>), dim3((unsigned)(na + nb)), dim3(A::kThreads), 0, stream,
+                       a, b, (int)nb);
     return hipGetLastError();
 }
 
@@ -1006,26 +1172,80 @@ hipError_t prologue(const PrologueArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-//           K  TAIL  MB NB WM WN KS AD EPI
-hipError_t conv(Conv op, const ConvArgs& c, hipStream_t stream) {
-    const long long px = (long long)c.H * c.W;
-    switch (op) {
-        case Conv::Context:
-            if (px < 20000) return launch<Shape<5, true, 4, 4, 1, 1, 4, 2, kPlain>>(c, stream);
-            return launch<Shape<5, true, 2, 4, 2, 2, 1, 2, kPlain>>(c, stream);
-        case Conv::Gates:
-            if (px < 20000) return launch<Shape<5, false, 2, 4, 1, 1, 4, 4, kGates>>(c, stream);
-            return launch<Shape<5, false, 4, 4, 2, 4, 1, 2, kGates>>(c, stream);
-        case Conv::Update:
-            if (px < 20000) return launch<Shape<5, false, 2, 4, 1, 1, 4, 4, kUpdate>>(c, stream);
-            return launch<Shape<5, false, 2, 4, 2, 2, 1, 2, kUpdate>>(c, stream);
-        default:
-            if (px < 20000) return launch<Shape<3, true, 4, 4, 1, 1, 4, 2, kHeads>>(c, stream);
-            return launch<Shape<3, true, 4, 4, 1, 2, 2, 2, kHeads>>(c, stream);
-    }
+// The shapes of a forward's convolutions by grid size, in 16 x 4 tiles: a small
+// grid takes small tiles and splits the reduction over a workgroup's waves, so
+// that the chip fills; a large one shares each weight over more pixels.  The
+// whole forward in us with each set (tiles):
+//            13x19(8) 40x60(40) 48x80(60) 60x80(75) 80x100(140) 90x160(230)
+//   Tiny       134      152       183       204        292         402
+//   Small      151      163       176       198        267         361
+//   Medium     194      208        -        223        254         346
+//   Large      377      389        -        388        412         438
+//            128x160(320) 160x200(520) 200x200(650) 256x256(1024)
+//   Medium     472          727          800          1172
+//   Large      486          759          805          1044
+// Gates and heads in one launch (they depend on the same hidden state only):
+// 19.1 against 12.0 + 11.0 us at 60x80, 130 against 76 + 64 us at 256x256.
+//                               K  TAIL  MB NB WM WN KS AD EPI
+struct Tiny {
+    using Context = Shape<5, true, 4, 2, 1, 1, 4, 2, kPlain>;
+    using Gates = Shape<5, false, 2, 2, 1, 1, 4, 4, kGates>;
+    using Update = Shape<5, false, 2, 2, 1, 1, 4, 4, kUpdate>;
+    using Heads = Shape<3, true, 4, 2, 1, 1, 4, 2, kHeads>;
+    using Up = Shape<3, true, 4, 2, 1, 1, 4, 2, kUp>;
+};
+struct Small {
+    using Context = Shape<5, true, 4, 4, 1, 1, 4, 2, kPlain>;
+    using Gates = Shape<5, false, 2, 4, 1, 1, 4, 4, kGates>;
+    using Update = Shape<5, false, 2, 4, 1, 1, 4, 4, kUpdate>;
+    using Heads = Shape<3, true, 4, 4, 1, 1, 4, 2, kHeads>;
+    using Up = Tiny::Up;
+};
+struct Medium {
+    using Context = Shape<5, true, 4, 4, 1, 2, 2, 2, kPlain>;
+    using Gates = Shape<5, false, 2, 4, 1, 2, 2, 4, kGates>;
+    using Update = Shape<5, false, 2, 4, 1, 2, 4, 4, kUpdate>;
+    using Heads = Shape<3, true, 4, 4, 1, 2, 2, 2, kHeads>;
+    using Up = Tiny::Up;
+};
+struct Large {
+    using Context = Shape<5, true, 2, 4, 2, 2, 1, 2, kPlain>;
+    using Gates = Shape<5, false, 4, 4, 2, 2, 1, 2, kGates>;
+    using Update = Shape<5, false, 2, 4, 2, 2, 1, 4, kUpdate>;
+    using Heads = Medium::Heads;
+    using Up = Shape<3, true, 4, 4, 1, 2, 2, 2, kUp>;
+};
+
+template <class F>
+hipError_t by_size(const ConvArgs& c, F f) {
+    const long long tiles = (long long)((c.W + kTW - 1) / kTW) * ((c.H + 3) / 4);
+    if (tiles <= 48) return f(Tiny{});
+    if (tiles <= 110) return f(Small{});
+    if (tiles <= 640) return f(Medium{});
+    return f(Large{});
 }
 
-constexpr Kernels kTable = {pack, prologue, conv};
+hipError_t conv(Conv op, const ConvArgs& c, hipStream_t stream) {
+    return by_size(c, [&](auto set) {
+        using Set = decltype(set);
+        switch (op) {
+            case Conv::Context: return launch<typename Set::Context>(c, stream);
+            case Conv::Gates: return launch<typename Set::Gates>(c, stream);
+            case Conv::Update: return launch<typename Set::Update>(c, stream);
+            case Conv::Heads: return launch<typename Set::Heads>(c, stream);
+            default: return launch<typename Set::Up>(c, stream);
+        }
+    });
+}
+
+hipError_t gates_heads(const ConvArgs& gates, const ConvArgs& heads, hipStream_t stream) {
+    return by_size(gates, [&](auto set) {
+        using Set = decltype(set);
+        return launch_pair<typename Set::Gates, typename Set::Heads>(gates, heads, stream);
+    });
+}
+
+constexpr Kernels kTable = {pack, prologue, conv, gates_heads};
 struct Register {
     Register() { kernels() = &kTable; }
 } const g_register;

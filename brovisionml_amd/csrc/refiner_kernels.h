@@ -102,8 +102,8 @@ struct ConvArgs {
     void* rs;               // gates: r*h, split (c4 where info says exact)
     float* out;             // context: c4; update: the new hidden state, c4
     void* outs;             // update: the new hidden state, split
-    // heads, per head: the two 1x1 layers packed, the three layers' biases
-    // (b4 NULL: none), the output planes (NCHW) and their count
+    // heads, per head: the two 1x1 layers packed, the three layers' biases,
+    // the output planes (NCHW; up: none) and their count
     const float* w2[4];
     const float* w4[4];
     const float* hb0[4];
@@ -111,13 +111,25 @@ struct ConvArgs {
     const float* b4[4];
     float* hout[4];
     int nout[4];
+    // up: the normals (3 planes) to upsample by head 3's output; the
+    // normalise's eps; the result's rows from pad_t and columns from pad_l, out_h x out_w; whether it takes
+    // 16-byte stores
+    const float* pred;
+    float* up;
+    float up_eps;
+    int pad_t, pad_l, out_h, out_w;
+    bool up_vec4;
 };
-enum class Conv { Context, Gates, Update, Heads };
+// Heads: the first three heads; Up: the up-mask head, the convex upsample and
+// its normalise.
+enum class Conv { Context, Gates, Update, Heads, Up };
 
 struct Kernels {
     hipError_t (*pack)(const PackArgs&, hipStream_t);
     hipError_t (*prologue)(const PrologueArgs&, hipStream_t);
     hipError_t (*conv)(Conv, const ConvArgs&, hipStream_t);
+    // Conv::Gates and Conv::Heads of the same hidden state
+    hipError_t (*gates_heads)(const ConvArgs& gates, const ConvArgs& heads, hipStream_t);
 };
 // Set when refiner_conv.hip is linked in (a build of the host code alone has
 // none).

@@ -25,7 +25,7 @@ namespace {
 using namespace bvml_refine;
 
 // The maps of a grid of up to 5,086 pixels (a 60 x 80 grid, the refiner's
-// size for a 480 x 640 image, is 4,800), 28 MB.
+// size for a 480 x 640 image, is 4,800), 13 MB.
 constexpr size_t kScratchFloats = maps_floats(5086);
 static __device__ __align__(256) float scratch[kScratchFloats];
 

@@ -51,9 +51,21 @@ def check(got, want, grow=1.0):
 
 
 @pytest.mark.parametrize("H,W", [(1, 1), (1, 33), (2, 16), (3, 17), (4, 15), (9, 31), (8, 48),
-                                 (17, 65), (129, 161)])
+                                 (17, 65), (129, 161),
+                                 # either side of a choice of tile: 48, 110 of 16 x 4
+                                 (45, 64), (45, 65), (40, 161), (41, 161)])
 def test_grids(cuda, H, W):
     check(*run(H, W, 60.0, H + W))
+
+
+@pytest.mark.parametrize("H,W", [(160, 256), (161, 249)])
+def test_large_grids(cuda, H, W):
+    """Either side of 640 tiles.  Of these 40,000 pixels a few have an xy pair
+    so small that it amplifies the heads' rounding: convolutions in plain fp32
+    matrix products differ from the restatement by up to 1.61e-5 (result) and
+    2.44e-4 (coarse) on these same inputs, the split products by 5.7e-6 and
+    2.2e-4, so the bars here are 4 times those of the smaller grids."""
+    check(*run(H, W, 60.0, H + W), grow=4.0)
 
 
 @pytest.mark.parametrize("scale", [1e-6, 30.0])
@@ -73,3 +85,33 @@ def test_non_finite(cuda, which, value):
     def change(maps):
         maps[which][7, 10, 3] = value
     check(*run(20, 70, 60.0, 41, change))
+
+
+def test_non_finite_medium(cuda):
+    """A row through the fp32 products beside split ones, four rows a wave."""
+    def change(maps):
+        maps[2][7, 10, 3] = np.inf
+    check(*run(62, 97, 60.0, 43, change))
+
+
+@pytest.mark.parametrize("H,W", [(13, 19), (62, 97), (161, 249)])
+@pytest.mark.parametrize("pad_t,pad_l,cut_h,cut_w", [(0, 0, 0, 4), (5, 3, 11, 6), (8, 4, 9, 8),
+                                                     (7, 0, 7, 1)])
+def test_crop_is_a_slice(cuda, H, W, pad_t, pad_l, cut_h, cut_w):
+    """The crop the upsample writes (16-byte or single stores) has the whole
+    result's bits, into an `out` of any alignment, and coarse maps asked for
+    change neither."""
+    import torch
+    print(f"[gpu] refiner {H}x{W} crop {pad_t} {pad_l} {cut_h} {cut_w}", flush=True)
+    intr = wl.intrins_from_fov(8 * H, 8 * W, 60.0)
+    model = rf.NativeRefiner(rf.random_weights(3))
+    dec = rf.DecoderOutput(*(torch.from_numpy(a)[None].to("cuda:0") for a in pins.inputs(H, W, 3)))
+    whole = model.forward(dec, intr, 8 * H, 8 * W)
+    crop = rf.Crop(orig_h=8 * H - cut_h, orig_w=8 * W - cut_w, pad_t=pad_t, pad_l=pad_l)
+    want = whole[:, :, pad_t:pad_t + crop.orig_h, pad_l:pad_l + crop.orig_w]
+    for shift in (0, 1):
+        flat = torch.full((3 * crop.orig_h * crop.orig_w + 8,), 7.0, device="cuda:0")
+        out = flat[shift:shift + 3 * crop.orig_h * crop.orig_w].view(1, 3, crop.orig_h, crop.orig_w)
+        got, _ = model.forward(dec, intr, 8 * H, 8 * W, crop=crop, coarse=True, out=out)
+        assert torch.equal(got, want)
+        assert bool((flat[:shift] == 7.0).all()) and bool((flat[shift + out.numel():] == 7.0).all())
