@@ -72,6 +72,10 @@ using bvml::Taps;
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 
+// Relative error of v_exp_f32 on [-126, 0], measured exhaustively (8.484e-8).
+constexpr float kExpRel = 8.5e-8f;
+static_assert(kExpRel == bvml::kExpRel, "the bound the sub-pixels use");
+
 // s = 8.  Block of 4 waves; wave gw = 8 * group + ky; lane = 2 * i + h owns
 // pixel group*32 + i and sub-pixels kx = 4h .. 4h + 3.
 constexpr int kLanesPerPx = 2;
