@@ -1185,7 +1185,7 @@ hipError_t prologue(const PrologueArgs& a, hipStream_t stream) {
 //   Medium     472          727          800          1172
 //   Large      486          759          805          1044
 // Gates and heads in one launch (they depend on the same hidden state only):
-// 19.1 against 12.0 + 11.0 us at 60x80, 130 against 76 + 64 us at 256x256.
+// 19.1 against 12.0 + 11.0 us at 60x80 (Small), 130 against 76 + 64 us at 256x256.
 //                               K  TAIL  MB NB WM WN KS AD EPI
 struct Tiny {
     using Context = Shape<5, true, 4, 2, 1, 1, 4, 2, kPlain>;
@@ -1200,6 +1200,13 @@ struct Small {
     using Update = Shape<5, false, 2, 4, 1, 1, 4, 4, kUpdate>;
     using Heads = Shape<3, true, 4, 4, 1, 1, 4, 2, kHeads>;
     using Up = Tiny::Up;
+};
+// Small's gates and heads are 7 workgroups a tile, and the chip holds 512 of
+// them: past 73 tiles gates of twice the channels (5 a tile) avoid a second,
+// nearly empty round (197 against 208 us at 60x80, 75 tiles; 187 against 180 at
+// 50x72, 65).
+struct SmallFull : Small {
+    using Gates = Shape<5, false, 4, 4, 1, 1, 4, 2, kGates>;
 };
 struct Medium {
     using Context = Shape<5, true, 4, 4, 1, 2, 2, 2, kPlain>;
@@ -1220,7 +1227,8 @@ template <class F>
 hipError_t by_size(const ConvArgs& c, F f) {
     const long long tiles = (long long)((c.W + kTW - 1) / kTW) * ((c.H + 3) / 4);
     if (tiles <= 48) return f(Tiny{});
-    if (tiles <= 110) return f(Small{});
+    if (tiles <= 73) return f(Small{});
+    if (tiles <= 110) return f(SmallFull{});
     if (tiles <= 640) return f(Medium{});
     return f(Large{});
 }

@@ -52,8 +52,8 @@ def check(got, want, grow=1.0):
 
 @pytest.mark.parametrize("H,W", [(1, 1), (1, 33), (2, 16), (3, 17), (4, 15), (9, 31), (8, 48),
                                  (17, 65), (129, 161),
-                                 # either side of a choice of tile: 48, 110 of 16 x 4
-                                 (45, 64), (45, 65), (40, 161), (41, 161)])
+                                 # either side of a choice of tile: 48, 73, 110 of 16 x 4
+                                 (45, 64), (45, 65), (72, 64), (73, 64), (40, 161), (41, 161)])
 def test_grids(cuda, H, W):
     check(*run(H, W, 60.0, H + W))
 
