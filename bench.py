@@ -1099,7 +1099,7 @@ def bench_refiner(args, dev) -> dict:
                      {"workload": f"dsine-refiner-{H}x{W}", "H": H, "W": W, "iterations": 5,
                       "weights": "synthetic (uniform +-1/sqrt(fan_in))",
                       "driver": driver,
-                      "convolutions": "5x5 and 3x3: implicit-GEMM fp32 MFMA kernels; the "
+                      "convolutions": "5x5 and 3x3: implicit-GEMM split-half f16 MFMA kernels, fp32 precision; the "
                                       "ConvGRU's parts over [feature, uv] once per forward"})
     if t_py is not None:
         line["python_driver"] = {"ms_per_step": round(t_py * 1e3 / args.steps, 4),

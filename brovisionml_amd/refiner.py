@@ -256,11 +256,11 @@ class Refiner:
 class NativeRefiner:
     """Refiner::forward in C++ (libbvml_dsine_refine.so, the C ABI of
     include/bvml_dsine_refine.h): the same loop as Refiner above, with no
-    Python or torch in it: the 5x5 ConvGRU convolutions on this package's
-    fp32 matrix-core kernels with the gates and update fused, the heads'
-    3x3 layer on the same kernels, the rest of the heads in one fused pass,
-    the rest this package's kernels, the up-mask head and the upsample in
-    the last iteration only: the same bits in every process.  Weights from a safetensors file (`path`, read by
+    Python or torch in it: the ConvGRU's 5x5 and the heads' 3x3 convolutions
+    on this package's split-half f16 matrix-core kernels at fp32 precision,
+    with the gates, the update and the rest of the heads in their epilogues,
+    the up-mask head with the upsample after the last iteration only: the
+    same bits in every process.  Weights from a safetensors file (`path`, read by
     the library) or a dict as weight_shapes() names them."""
 
     def __init__(self, weights: dict | None = None, path: str | None = None):
