@@ -689,6 +689,7 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     pa.ray = m.ray; pa.uv = m.uv; pa.pred = m.pred[0];
     pa.hf = m.hf; pa.hs = m.hs; pa.fs = m.fs;
     pa.th = reinterpret_cast<uint32_t*>(m.th); pa.tf = reinterpret_cast<uint32_t*>(m.tf);
+    pa.w_q = r->w_q;
     pa.info = reinterpret_cast<uint32_t*>(m.info);
     if ((st = hip(kern->prologue(pa, strm), "prologue"))) return st;
     // the ConvGRU convolutions' parts over [feature | uv], which no
@@ -696,7 +697,7 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     ConvArgs base{};
     base.info = pa.info; base.uv = m.uv; base.H = h8; base.W = w8;
     ConvArgs ctx = base;
-    ctx.xs = m.fs; ctx.x32 = m.fs; ctx.tail = pa.tf; ctx.which = 1;
+    ctx.xs = m.fs; ctx.x32 = a.feature; ctx.tail = pa.tf; ctx.which = 1;
     ctx.wp = r->w_ctx; ctx.cout = ctx.wcout = 3 * kHidden; ctx.out = m.cf;
     if ((st = hip(kern->conv(Conv::Context, ctx, strm), "context convolution"))) return st;
     // the ConvGRU (:138-159): the 5x5 convolutions over h (r*h) plus their

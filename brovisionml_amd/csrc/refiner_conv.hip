@@ -328,7 +328,9 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
 
     if constexpr (EARLY) epilogue_loads();
     const int xn = info->n[c.which];
-    const bool exact = info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
+    // (the update reads r*h in the form that the gates wrote)
+    const bool exact = EPI == kUpdate ? info->rh32 != 0
+                                      : info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
     __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
     __syncthreads();
 
@@ -405,7 +407,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
             }
         }
     } else {
-        // fp32 products of the c4 map and the unsplit weights: one 16x16x4
+        // fp32 products of the fp32 map and the unsplit weights: one 16x16x4
         // step per tap and 4 channels
         constexpr int GROUPS = split_groups(TAIL);
         const float* const w32 = c.wp + whead + (size_t)a.wblocks * STEPS * 512;
@@ -421,8 +423,9 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                     const int y = ty0 + wn * NB + n + tap / K - P, x = tx0 + col + tap % K - P;
                     const bool in = y >= 0 && y < H && x >= 0 && x < W && !(tail && g >= 2);
                     const size_t px = in ? (uint32_t)(y * W + x) : 0u;
-                    const float f = !TAIL || !tail ? c.x32[((size_t)cg * HW + px) * 4 + g]
-                                                   : c.uv[(g < 2 ? g : 0) * HW + px];
+                    const float f = TAIL && tail ? c.uv[(g < 2 ? g : 0) * HW + px]
+                                    : EPI == kPlain ? c.x32[((size_t)4 * cg + g) * HW + px]
+                                                    : c.x32[((size_t)cg * HW + px) * 4 + g];
                     const float bf = in ? f : 0.0f;
 #pragma unroll
                     for (int m = 0; m < MB; ++m)
@@ -872,7 +875,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                             ep[2][j][p][r];
                 }
                 *reinterpret_cast<v4f*>(c.z + c4_at(q0 + p, px)) = zz;
-                if (info->exact[0])
+                if (info->rh32)
                     *reinterpret_cast<v4f*>(static_cast<float*>(c.rs) + c4_at(q0 + p, px)) = rh;
                 else
                     store_split(c.rs, q0 + p, px, rh);
@@ -1115,6 +1118,8 @@ __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, 
             info->n[k] = n[k];
             info->exact[k] = exact[k];
         }
+        const int* const q = reinterpret_cast<const int*>(a.w_q);
+        info->rh32 = exact[0] || q[64] == 0;  // (the flag behind 64 exponents)
     }
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (blockIdx.y == 2) {
@@ -1139,9 +1144,8 @@ __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, 
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = src[(size_t)j * HW];
-    float* c4 = k == 0 ? a.hf : (exact[1] ? a.fs : nullptr);
-    if (c4) {
-        v4f* d = reinterpret_cast<v4f*>(c4);
+    if (k == 0) {
+        v4f* d = reinterpret_cast<v4f*>(a.hf);
         d[(size_t)(2 * grp) * HW + px] = v4f{v[0], v[1], v[2], v[3]};
         d[(size_t)(2 * grp + 1) * HW + px] = v4f{v[4], v[5], v[6], v[7]};
     }

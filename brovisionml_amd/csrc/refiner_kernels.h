@@ -23,7 +23,9 @@ namespace bvml_refine {
 // r*h and the uv tail beside h), 1: the feature map's (and the tail beside it).
 struct Info {
     int n[2];      // scale exponents
-    int exact[2];  // 1: an operand has no usable scale, convolve c4 maps in fp32
+    int exact[2];  // 1: an operand has no usable scale, convolve fp32 maps in fp32
+    int rh32;      // 1: r*h is c4, not split: exact[0], or convq's weights over it have an
+                   // infinity or a NaN (the update then takes the fp32 products)
 };
 constexpr int kMaxBlocks = 256;  // partial maxima of each map
 constexpr size_t kInfoWords = 64 + 2 * kMaxBlocks;
@@ -73,8 +75,7 @@ struct PackArgs {
 };
 
 // The first steps of a forward: ray and uv maps, pred = RayReLU(normal, ray),
-// the scales, hidden as hf (c4) and hs (split), feature as fs (split, or c4
-// where info says exact), the tails.
+// the scales, hidden as hf (c4) and hs (split), feature as fs (split), the tails.
 struct PrologueArgs {
     const float *normal, *hidden, *feature;  // 3, 64 and 64 planes
     double fu, cu, fv, cv;
@@ -82,13 +83,14 @@ struct PrologueArgs {
     float *ray, *uv, *pred;     // 3, 2 and 3 planes
     float *hf, *hs, *fs;        // 64-channel maps
     uint32_t *th, *tf;          // tails
+    const float* w_q;           // the update's packed weights, kHidden channels
     uint32_t* info;             // kInfoWords: Info, then (from word 64) partial maxima
 };
 
 // One convolution.
 struct ConvArgs {
     const void* xs;         // split map, 64 channels
-    const float* x32;       // the same map in c4, read where info says exact
+    const float* x32;       // the same map in fp32, for the fp32 products: c4 (context: NCHW)
     const uint32_t* tail;   // tail, or NULL
     const float* uv;        // the tail's planes in fp32 (exact)
     const uint32_t* info;
@@ -99,7 +101,7 @@ struct ConvArgs {
     const float *b0, *b1;   // biases: gates z and r; update q
     const float* hf;        // gates, update: the hidden state, c4
     float* z;               // c4: gates write it, update reads it
-    void* rs;               // gates: r*h, split (c4 where info says exact)
+    void* rs;               // gates: r*h, split (c4 where info says rh32)
     float* out;             // context: c4; update: the new hidden state, c4
     void* outs;             // update: the new hidden state, split
     // heads, per head: the two 1x1 layers packed, the three layers' biases,

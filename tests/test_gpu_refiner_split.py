@@ -19,11 +19,13 @@ pytestmark = pytest.mark.gpu
 TOL_RESULT, TOL_COARSE = 5e-6, 1e-4
 
 
-def run(H, W, fov, seed, change=None):
+def run(H, W, fov, seed, change=None, change_weights=None):
     """(native result, coarse), (restatement's result, coarse)."""
     import torch
     print(f"[gpu] refiner {H}x{W} fov {fov}", flush=True)
     weights = rf.random_weights(seed)
+    if change_weights:
+        change_weights(weights)
     maps = [a.copy() for a in pins.inputs(H, W, seed)]
     if change:
         change(maps)
@@ -94,6 +96,44 @@ def test_non_finite_medium(cuda):
     def change(maps):
         maps[2][7, 10, 3] = np.inf
     check(*run(62, 97, 60.0, 43, change))
+
+
+# (max-abs, rms) of result and coarse that convolutions in plain fp32 matrix
+# products (csrc/conv.hip) show against the restatement, at most, over the
+# inputs of the tests that use them: a pixel with a small xy pair amplifies its
+# heads' rounding, so the rms says more.  The bars are four times these.
+FP32_INFINITE = ((1.44e-5, 4.7e-7), (7.44e-4, 3.4e-6))
+
+
+def check_fp32(got, want, fp32):
+    for g, w, (mx, rms) in zip(got, want, fp32):
+        assert np.array_equal(np.isnan(g), np.isnan(w))
+        d = np.abs(g - w)[~np.isnan(w)]
+        print(f"    max-abs {d.max(initial=0.0):.3e}, rms {np.sqrt((d ** 2).sum() / max(1, d.size)):.3e}, "
+              f"{np.isnan(w).mean():.3f} NaN", flush=True)
+        assert d.max(initial=0.0) <= 4 * mx
+        assert (d ** 2).sum() <= (4 * rms) ** 2 * d.size
+
+
+INFINITE = [
+    ("gru.convz.weight", (5, 90, 2, 2)), ("gru.convz.weight", (5, 129, 2, 2)),
+    ("gru.convr.weight", (17, 3, 2, 2)), ("gru.convq.weight", (5, 9, 2, 2)),
+    ("gru.convq.weight", (63, 64, 2, 2)), ("gru.convq.weight", (9, 20, 0, 4)),
+    ("xy_head.0.weight", (3, 7, 1, 1)), ("angle_head.2.weight", (0, 63, 0, 0)),
+    ("up_prob_head.0.weight", (8, 65, 1, 1)), ("prob_head.4.weight", (24, 1, 0, 0))]
+
+
+@pytest.mark.parametrize("H,W,name,at", [(20, 70, *i) for i in INFINITE] +
+                         [(62, 97, *i) for i in INFINITE if "gru" in i[0]] +
+                         [(161, 256, *i) for i in INFINITE[1:6:2]])
+def test_infinite_weight(cuda, H, W, name, at):
+    """One infinite weight beside finite maps, in each part of each layer: it
+    saturates (or makes NaN) what it reaches and no more.  (At the centre tap
+    no padding zero meets it; the one in a corner makes NaN at the border,
+    which spreads.)"""
+    def change(w):
+        w[name][at] = np.inf
+    check_fp32(*run(H, W, 60.0, 41, change_weights=change), FP32_INFINITE)
 
 
 @pytest.mark.parametrize("H,W", [(13, 19), (62, 97), (161, 249)])
