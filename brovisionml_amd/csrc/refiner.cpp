@@ -689,7 +689,9 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     pa.ray = m.ray; pa.uv = m.uv; pa.pred = m.pred[0];
     pa.hf = m.hf; pa.hs = m.hs; pa.fs = m.fs;
     pa.th = reinterpret_cast<uint32_t*>(m.th); pa.tf = reinterpret_cast<uint32_t*>(m.tf);
-    pa.w_q = r->w_q;
+    pa.w_ctx = r->w_ctx; pa.w_zr = r->w_zr; pa.w_q = r->w_q; pa.w_h0 = r->w_h0;
+    pa.mb_ctx = 3 * kHidden / 16; pa.mb_zr = 2 * kHidden / 16; pa.mb_q = kHidden / 16;
+    pa.mb_h0 = kHeads * kMid / 16;
     pa.info = reinterpret_cast<uint32_t*>(m.info);
     if ((st = hip(kern->prologue(pa, strm), "prologue"))) return st;
     // the ConvGRU convolutions' parts over [feature | uv], which no
@@ -707,8 +709,9 @@ int bvml_refine::forward_maps(bvml_dsine_refiner* r, const Maps& m, const Forwar
     gates.xs = m.hs; gates.x32 = m.hf; gates.wp = r->w_zr; gates.cout = gates.wcout = 2 * kHidden;
     gates.s0 = m.cf; gates.b0 = r->b_z; gates.b1 = r->b_r; gates.hf = m.hf; gates.z = m.z;
     gates.rs = m.rs;
+    gates.rh32 = m.fs;  // (the context was its only reader)
     ConvArgs update = base;
-    update.xs = m.rs; update.x32 = m.rs; update.wp = r->w_q; update.cout = update.wcout = kHidden;
+    update.xs = m.rs; update.x32 = m.fs; update.wp = r->w_q; update.cout = update.wcout = kHidden;
     update.s0 = m.cf + (size_t)2 * kHidden * hw; update.b0 = r->b_q; update.hf = m.hf;
     update.z = m.z; update.out = m.hf; update.outs = m.hs;
     // the heads the propagate reads (:119-127, :257-267)

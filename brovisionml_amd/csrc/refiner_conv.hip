@@ -3,18 +3,20 @@
 // fused (src/dsine_refine.cpp:119-159), and the first steps of a forward.
 //
 // The convolutions are implicit GEMMs on the f16 matrix cores at fp32
-// precision.  Every operand, scaled by a power of two, is the sum of two
-// halfs, hi = half(v) and lo = half(v - hi), to within 2^-23 of itself; a
-// product is three matrix-core products (hi hi + hi lo + lo hi; the omitted
-// lo lo is at most 2^-22 of it) summed in fp32.  The weights are split when
-// they are packed, each output channel scaled to its largest weight; a map is
-// split by the kernel that writes it, scaled to a bound of its values: the
-// largest feature, and for the hidden state the largest of 1 and the decoder's
-// |hidden| (a ConvGRU state never exceeds it).  A value is kept to full
-// precision down to 2^-29 of the bound, and none is off by more than 2^-39 of
-// it.  The scales come off the sums exactly.  Where an operand has no such
-// scale (an infinity, a NaN, magnitudes from 2^64) the same kernels convolve
-// the fp32 maps on the fp32 matrix cores.
+// precision.  Every operand, scaled by a power of two to below 2^15, is the
+// sum of two halfs, hi = half(v) and lo = half(v - hi); a product is three
+// matrix-core products (hi hi + hi lo + lo hi; the omitted lo lo is at most
+// 2^-22 of it) summed in fp32.  A value is off by at most 2^-23 of itself down
+// to 2^-16 of its scale's bound, below that by at most 2^-39 of the bound.  The
+// scales come off the sums exactly.  The weights are split when they are
+// packed, each output channel scaled to its largest weight; a map is split by
+// the kernel that writes it, by one scale: that of its largest value (of the
+// hidden state: the largest of 1 and the decoder's |hidden|, which a ConvGRU
+// state never exceeds), but no larger than leaves the sums as precise as the
+// activations they go to can use (kBudget).  A value beyond that scale, an
+// infinity or a NaN makes the sums of the windows that hold it infinite or NaN,
+// and the workgroups that find such sums convolve the fp32 maps on the fp32
+// matrix cores instead, as all do whose weights have an infinity or a NaN.
 //
 // Three v_mfma_f32_16x16x32_f16 (16 cycles each) do the work of eight
 // v_mfma_f32_16x16x4_f32 (32 cycles each), and the sums' chains are shorter
@@ -76,6 +78,18 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t m) {
 }
 
 constexpr uint32_t kInfBits = 0x7f800000u;
+
+// Where a map's scale ends: its bound, times the largest weight of the layers
+// that read it, is at most 2^(kBudget + 1).  A value below the bound is off by at
+// most 2^-40 of it, so a sum of 1,650 products with weights spread up to the
+// largest by about 2^-40 2^9 sqrt(1650) / 3 = 2^-27 (rms), below the rounding of
+// a gate's argument of unit scale.  Values up to 2^13 times unit scale fit
+// beside weights of the usual +-1/sqrt(fan_in).
+constexpr int kBudget = 8;
+__device__ __forceinline__ uint32_t limit_bits(uint32_t wmax) {
+    const int e = 2 * 127 + kBudget - (int)(wmax >> 23);  // (at least 8: wmax is finite)
+    return (uint32_t)(e < 191 ? e : 191) << 23;
+}
 
 // The power of two that brings a magnitude of these bits into [2^14, 2^15),
 // as its exponent (at most 126, so that it is a normal float: a magnitude
@@ -140,7 +154,8 @@ struct Shape {
     // the up-mask head's normals, with a border of one pixel
     static constexpr int kPredAt = kParamAt + kParamBytes;
     static constexpr int kPredBytes = EPI == kUp ? (TH + 2) * (kTW + 2) * 16 : 0;
-    static constexpr int kLdsBytes = kPredAt + kPredBytes;
+    static constexpr int kRedoAt = kPredAt + kPredBytes;
+    static constexpr int kLdsBytes = kRedoAt + 16;
     static constexpr int NC = NB >= KS ? NB / KS : 1;  // columns (tile rows) a wave finishes
     static_assert(NB % KS == 0 || NB < KS, "whole columns per group");
     static_assert(AD % 2 == 0, "B operands alternate between two slots");
@@ -328,9 +343,10 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
 
     if constexpr (EARLY) epilogue_loads();
     const int xn = info->n[c.which];
-    // (the update reads r*h in the form that the gates wrote)
-    const bool exact = EPI == kUpdate ? info->rh32 != 0
-                                      : info->exact[c.which] != 0 || wexp[16 * a.wblocks] == 0;
+    const bool wide = info->wide[c.which] != 0;
+    bool exact = (uint32_t)wexp[16 * a.wblocks] >= kInfBits;  // fp32 products
+    int* const redo = reinterpret_cast<int*>(lds + S::kRedoAt);
+    if (KS > 1 && tid == 0) *redo = exact;
     __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
     __syncthreads();
 
@@ -406,7 +422,49 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                 products(0, 0);
             }
         }
-    } else {
+        // a window holds a value beyond the scale, an infinity or a NaN
+        if (wide) {
+            bool bad = false;
+#pragma unroll
+            for (int m = 0; m < MB; ++m)
+#pragma unroll
+                for (int n = 0; n < NB; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bad |= absbits(acc[m][n][r]) >= kInfBits;
+            exact = __any(bad);
+            if (KS > 1 && exact && lane == 0) *redo = 1;
+        }
+    }
+
+    // the heads' second layer's weights, in flight through what follows
+    constexpr uint32_t kHead64 = split1x1_head_words(64);
+    h8 w2v[HEAD ? 4 : 1][2][2];
+    auto w_load = [&](__amdgpu_buffer_rsrc_t rr, int ob, h8 (&w)[2][2]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            w[q][0] = ld16(rr, lane16, (uint32_t)(ob * 2 + q) * 2048u);
+            w[q][1] = ld16(rr, lane16 + 1024u, (uint32_t)(ob * 2 + q) * 2048u);
+        }
+    };
+    const int hd = EPI == kUp ? 3 : HEAD ? mg * WM + wm : 0;
+    auto w2_load = [&]() {
+        if constexpr (HEAD) {
+            const __amdgpu_buffer_rsrc_t r2 = rsrc_of(c.w2[hd] + kHead64, 4 * 2 * 2048u);
+#pragma unroll
+            for (int mo = 0; mo < 4; ++mo) w_load(r2, mo, w2v[mo]);
+        }
+    };
+    w2_load();
+
+    if constexpr (KS > 1) {
+        __syncthreads();  // every wave is done with the halo
+        exact = *redo != 0;  // (the waves that split the reduction, together)
+    }
+    if (exact) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         // fp32 products of the fp32 map and the unsplit weights: one 16x16x4
         // step per tap and 4 channels
         constexpr int GROUPS = split_groups(TAIL);
@@ -434,29 +492,12 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                 }
             }
         }
-    }
-
-    // the heads' second layer's weights, in flight through what follows
-    constexpr uint32_t kHead64 = split1x1_head_words(64);
-    h8 w2v[HEAD ? 4 : 1][2][2];
-    auto w_load = [&](__amdgpu_buffer_rsrc_t rr, int ob, h8 (&w)[2][2]) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            w[q][0] = ld16(rr, lane16, (uint32_t)(ob * 2 + q) * 2048u);
-            w[q][1] = ld16(rr, lane16 + 1024u, (uint32_t)(ob * 2 + q) * 2048u);
-        }
-    };
-    const int hd = EPI == kUp ? 3 : HEAD ? mg * WM + wm : 0;
-    if constexpr (HEAD) {
-        const __amdgpu_buffer_rsrc_t r2 = rsrc_of(c.w2[hd] + kHead64, 4 * 2 * 2048u);
-#pragma unroll
-        for (int mo = 0; mo < 4; ++mo) w_load(r2, mo, w2v[mo]);
+        w2_load();  // (so that they need no registers in these loops)
     }
 
     // the groups' partial sums meet: group ks finishes columns n = ks, ks + KS, ...
     v4f own[MB][NC];
     if constexpr (KS > 1) {
-        __syncthreads();  // every wave is done with the halo
         v4f* const xch =
             reinterpret_cast<v4f*>(lds) + (size_t)(wn * WM + wm) * (KS - 1) * MB * NB * 64 + lane;
         // column n, block m: the partials of the groups that do not own it
@@ -532,8 +573,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         const int nout = c.nout[hd], nob = (nout + 15) / 16;
         const uint32_t head4 = split1x1_head_words(nout);
         const __amdgpu_buffer_rsrc_t r4 = rsrc_of(w4 + head4, (uint32_t)nob * 2 * 2048u);
-        const bool ok2 = reinterpret_cast<const int*>(w2)[64] != 0;
-        const bool ok4 = reinterpret_cast<const int*>(w4)[16 * nob] != 0;
+        const bool ok2 = reinterpret_cast<const uint32_t*>(w2)[64] < kInfBits;
+        const bool ok4 = reinterpret_cast<const uint32_t*>(w4)[16 * nob] < kInfBits;
         auto exact16 = [&](const float* w32, int ob, const v4f (&v)[4]) {
             v4f o = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -875,10 +916,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                             ep[2][j][p][r];
                 }
                 *reinterpret_cast<v4f*>(c.z + c4_at(q0 + p, px)) = zz;
-                if (info->rh32)
-                    *reinterpret_cast<v4f*>(static_cast<float*>(c.rs) + c4_at(q0 + p, px)) = rh;
-                else
-                    store_split(c.rs, q0 + p, px, rh);
+                store_split(c.rs, q0 + p, px, rh);
+                if (info->rh32) *reinterpret_cast<v4f*>(c.rh32 + c4_at(q0 + p, px)) = rh;
             }
         }
     } else {
@@ -897,7 +936,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                     hn[r] = gru_mix(ep[1][j][m][r], ep[2][j][m][r],
                                     tanhf(own[m][j][r] + ep[0][j][m][r] + eb[0][m][r]));
                 *reinterpret_cast<v4f*>(c.out + c4_at(mb0 + m, px)) = hn;
-                if (!info->exact[0]) store_split(c.outs, mb0 + m, px, hn);
+                store_split(c.outs, mb0 + m, px, hn);
             }
         }
     }
@@ -982,13 +1021,12 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
         if (rowp[r]) atomicMax(&rowmax[r], absbits(rowp[r][i - r * cols]));
     }
     __syncthreads();
-    // [exponents | flag], the flag cleared by any block that finds an infinity
-    // or a NaN (it is set before these launches)
+    // [exponents | the largest] (0 before this launch)
     int* const head = reinterpret_cast<int*>(a.wp);
     if (tid < 16) {
         const uint32_t m = rowmax[tid];
         head[16 * mb + tid] = m < kInfBits ? -scale_exp(m) : 0;
-        if (m >= kInfBits) head[16 * nmb] = 0;
+        atomicMax(reinterpret_cast<uint32_t*>(head) + 16 * nmb, m);
     }
     const bool tail = cin > 64;
     const int steps = one ? 2 : split_steps(a.k, tail);
@@ -1027,11 +1065,11 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
     }
 }
 
-__global__ void pack_flag_kernel(float* wp, int nmb) { reinterpret_cast<int*>(wp)[16 * nmb] = 1; }
+__global__ void pack_zero_kernel(float* wp, int nmb) { reinterpret_cast<int*>(wp)[16 * nmb] = 0; }
 
 hipError_t pack(const PackArgs& a, hipStream_t stream) {
     const int nmb = (a.out + 15) / 16;
-    hipLaunchKernelGGL(pack_flag_kernel, dim3(1), dim3(1), 0, stream, a.wp, nmb);
+    hipLaunchKernelGGL(pack_zero_kernel, dim3(1), dim3(1), 0, stream, a.wp, nmb);
     hipLaunchKernelGGL(pack_kernel, dim3((unsigned)nmb), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
@@ -1041,8 +1079,6 @@ hipError_t pack(const PackArgs& a, hipStream_t stream) {
 // of the decoder's normals and the maps' largest magnitudes; then the scales
 // from those and the split maps.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kExactBits = 0x5f800000u;  // 2^64
-
 __global__ __launch_bounds__(256) void camera_kernel(PrologueArgs a, bool vec4) {
     const uint32_t HW = (uint32_t)a.H * (uint32_t)a.W;
     const uint32_t tid = blockIdx.x * 256u + threadIdx.x, nt = gridDim.x * 256u;
@@ -1094,6 +1130,16 @@ __global__ __launch_bounds__(256) void camera_kernel(PrologueArgs a, bool vec4) 
 // |u|, |v| of the map.
 __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, float uvmax) {
     const uint32_t HW = (uint32_t)a.H * (uint32_t)a.W;
+    // the largest weight of the layers that read each map (one with an infinity
+    // or a NaN takes fp32 products whatever the scale)
+    auto largest = [](const float* w, int mb) {
+        return reinterpret_cast<const uint32_t*>(w)[16 * mb];
+    };
+    auto finite = [](uint32_t m) { return m < kInfBits ? m : 0u; };
+    const uint32_t wq = largest(a.w_q, a.mb_q);
+    const uint32_t wmax[2] = {umax(umax(finite(largest(a.w_zr, a.mb_zr)), finite(wq)),
+                                   finite(largest(a.w_h0, a.mb_h0))),
+                              finite(largest(a.w_ctx, a.mb_ctx))};
     __shared__ uint32_t red[2][4];
     uint32_t mx[2];
     for (int k = 0; k < 2; ++k) {
@@ -1102,24 +1148,21 @@ __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, 
         if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = m;
     }
     __syncthreads();
-    int n[2], exact[2];
+    int n[2], wide[2];
     for (int k = 0; k < 2; ++k) {
         mx[k] = umax(umax(red[k][0], red[k][1]), umax(red[k][2], red[k][3]));
-        const uint32_t one = absbits(1.0f);
-        const uint32_t scale = umax(k == 0 ? umax(mx[k], one) : mx[k], absbits(uvmax));
-        n[k] = scale_exp(scale);
-        // (a uv map far beyond the maps it joins would take their precision)
-        exact[k] = mx[k] >= kExactBits ||
-                   !(uvmax <= 64.0f * __builtin_bit_cast(float, umax(mx[k], one)));
+        const uint32_t all = umax(k == 0 ? umax(mx[k], absbits(1.0f)) : mx[k], absbits(uvmax));
+        const uint32_t limit = limit_bits(wmax[k]) - 1;
+        n[k] = scale_exp(all < limit ? all : limit);
+        wide[k] = all > limit;
     }
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         Info* info = reinterpret_cast<Info*>(a.info);
         for (int k = 0; k < 2; ++k) {
             info->n[k] = n[k];
-            info->exact[k] = exact[k];
+            info->wide[k] = wide[k];
         }
-        const int* const q = reinterpret_cast<const int*>(a.w_q);
-        info->rh32 = exact[0] || q[64] == 0;  // (the flag behind 64 exponents)
+        info->rh32 = wide[0] || wq >= kInfBits;
     }
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (blockIdx.y == 2) {
@@ -1149,7 +1192,6 @@ __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, 
         d[(size_t)(2 * grp) * HW + px] = v4f{v[0], v[1], v[2], v[3]};
         d[(size_t)(2 * grp + 1) * HW + px] = v4f{v[4], v[5], v[6], v[7]};
     }
-    if (exact[k]) return;
     const float sc = pow2(n[k]);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] *= sc;

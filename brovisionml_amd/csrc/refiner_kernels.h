@@ -7,7 +7,8 @@
 //          as an accumulator block's lane holds them
 //   split  halfs, [hi, lo][C / 8][HW][8]: a pixel's 8 consecutive channels in
 //          16 bytes, as a matrix-core operand's lane takes them; a value v is
-//          (hi + lo) 2^-n with n the map's scale exponent (Info)
+//          (hi + lo) 2^-n with n the map's scale exponent (Info); hi is not
+//          finite where v 2^n rounds to 2^16 or more, or is not finite itself
 //   tail   halfs, [hi, lo][HW][2]: the uv planes at a split map's scale
 // A split map takes the bytes of the fp32 map.
 #pragma once
@@ -22,10 +23,9 @@ namespace bvml_refine {
 // Per-forward values on the device.  index 0: the hidden state's maps (h,
 // r*h and the uv tail beside h), 1: the feature map's (and the tail beside it).
 struct Info {
-    int n[2];      // scale exponents
-    int exact[2];  // 1: an operand has no usable scale, convolve fp32 maps in fp32
-    int rh32;      // 1: r*h is c4, not split: exact[0], or convq's weights over it have an
-                   // infinity or a NaN (the update then takes the fp32 products)
+    int n[2];     // scale exponents
+    int wide[2];  // 1: a split map may hold values that are not finite
+    int rh32;     // 1: the gates write r*h as c4 too: the update may need fp32 products
 };
 constexpr int kMaxBlocks = 256;  // partial maxima of each map
 constexpr size_t kInfoWords = 64 + 2 * kMaxBlocks;
@@ -33,8 +33,9 @@ constexpr size_t kInfoWords = 64 + 2 * kMaxBlocks;
 // Packed weights, in 32-bit words (pack).  A convolution over 64 channels (and a
 // tail of 2), 16-channel M-blocks mb:
 //   [16 mblocks] each output channel's scale exponent e: its weights times
-//     2^-e are below 2^15; then one flag, 0 where a weight is infinite or NaN;
-//     padded to a multiple of 64 words
+//     2^-e are below 2^15; then the bits of the layer's largest magnitude
+//     (from 0x7f800000 on: an infinity or a NaN); padded to a multiple of 64
+//     words
 //   [mb][step][hi, lo][64 lanes][8 halfs] the split weights: lane l holds
 //     output channel 16 mb + l % 16 and, in step c k^2 + tap (c = 0, 1),
 //     channels 32 c + 8 (l / 16) + j; in the tail's steps, which come last,
@@ -44,7 +45,7 @@ constexpr size_t kInfoWords = 64 + 2 * kMaxBlocks;
 //     with zeros where the row or column lies outside the kernel
 //   [mb][4-channel group][tap][64 lanes] the same in fp32: lane l holds output
 //     channel 16 mb + l % 16, channel 4 group + l / 16
-// A 64-input 1x1 layer: the exponents and the flag, [ob][q 0, 1][hi, lo][64][8
+// A 64-input 1x1 layer: the exponents and the largest, [ob][q 0, 1][hi, lo][64][8
 // halfs] with lane l holding output 16 ob + l % 16, input
 // 16 (2 q + j / 4) + 4 (l / 16) + j % 4 (the accumulators of two M-blocks as
 // they stand), then [ob][m 4][r 4][64 lanes] in fp32, lane l holding output
@@ -83,14 +84,18 @@ struct PrologueArgs {
     float *ray, *uv, *pred;     // 3, 2 and 3 planes
     float *hf, *hs, *fs;        // 64-channel maps
     uint32_t *th, *tf;          // tails
-    const float* w_q;           // the update's packed weights, kHidden channels
+    // the packed layers that read the features (ctx) and the hidden state, and
+    // their 16-channel blocks
+    const float *w_ctx, *w_zr, *w_q, *w_h0;
+    int mb_ctx, mb_zr, mb_q, mb_h0;
     uint32_t* info;             // kInfoWords: Info, then (from word 64) partial maxima
 };
 
 // One convolution.
 struct ConvArgs {
     const void* xs;         // split map, 64 channels
-    const float* x32;       // the same map in fp32, for the fp32 products: c4 (context: NCHW)
+    const float* x32;       // the same map in fp32, for the fp32 products: c4 (context: NCHW;
+                            // update: written where info says rh32)
     const uint32_t* tail;   // tail, or NULL
     const float* uv;        // the tail's planes in fp32 (exact)
     const uint32_t* info;
@@ -101,7 +106,8 @@ struct ConvArgs {
     const float *b0, *b1;   // biases: gates z and r; update q
     const float* hf;        // gates, update: the hidden state, c4
     float* z;               // c4: gates write it, update reads it
-    void* rs;               // gates: r*h, split (c4 where info says rh32)
+    void* rs;               // gates: r*h, split
+    float* rh32;            // gates: r*h, c4 (where info says rh32)
     float* out;             // context: c4; update: the new hidden state, c4
     void* outs;             // update: the new hidden state, split
     // heads, per head: the two 1x1 layers packed, the three layers' biases,

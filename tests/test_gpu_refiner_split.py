@@ -2,10 +2,11 @@
 split-half matrix products at fp32 precision) against the float64 restatement
 (oracle/refiner.py), where their tiling, their scales and their fp32 path can
 go wrong: grids around the tile sizes, one-pixel grids, hidden states far from
-unit scale, a field of view whose uv map leaves the split form's range, an
-infinity or a NaN in the decoder's maps.  The bars are those of
-tests/test_gpu_refiner_native.py; a map with a non-finite value has the
-restatement's NaN pattern and its values elsewhere."""
+unit scale, maps and weights of opposite scales, single values beyond a split
+map's scale, a uv map beyond it, an infinity or a NaN in the decoder's maps or
+in a weight.  The bars are those of tests/test_gpu_refiner_native.py, or four
+times what plain fp32 convolutions show on the same inputs; non-finite values
+give the restatement's NaN pattern and its values elsewhere."""
 from __future__ import annotations
 
 import numpy as np
@@ -19,16 +20,16 @@ pytestmark = pytest.mark.gpu
 TOL_RESULT, TOL_COARSE = 5e-6, 1e-4
 
 
-def run(H, W, fov, seed, change=None, change_weights=None):
+def run(H, W, fov, seed, change=lambda maps: None, change_weights=lambda w: None,
+        change_both=lambda maps, w: None):
     """(native result, coarse), (restatement's result, coarse)."""
     import torch
     print(f"[gpu] refiner {H}x{W} fov {fov}", flush=True)
     weights = rf.random_weights(seed)
-    if change_weights:
-        change_weights(weights)
     maps = [a.copy() for a in pins.inputs(H, W, seed)]
-    if change:
-        change(maps)
+    change(maps)
+    change_weights(weights)
+    change_both(maps, weights)
     intr = wl.intrins_from_fov(8 * H, 8 * W, fov)
     dec = rf.DecoderOutput(*(torch.from_numpy(a)[None].to("cuda:0") for a in maps))
     out, coarse = rf.NativeRefiner(weights).forward(dec, intr, 8 * H, 8 * W, coarse=True)
@@ -50,6 +51,27 @@ def check(got, want, grow=1.0):
         err = np.nanmax(np.abs(g - w), initial=0.0)
         print(f"    max-abs {err:.3e}, {np.isnan(w).mean():.3f} NaN", flush=True)
         assert err <= grow * tol
+
+
+# (max-abs, rms) of result and coarse that convolutions in plain fp32 matrix
+# products (csrc/conv.hip) show against the restatement, at most, over the
+# inputs of the tests that use them: a pixel with a small xy pair amplifies its
+# heads' rounding, so the rms says more.  The bars are four times these.
+FP32_INFINITE = ((1.44e-5, 4.7e-7), (7.44e-4, 3.4e-6))
+FP32_SPREAD = ((2.24e-5, 4.9e-7), (4.46e-4, 1.03e-6))
+FP32_SCALE = ((3.72e-6, 4.7e-7), (1.83e-5, 1.0e-6))
+FP32_WIDE = {179.8: ((1.44e-5, 1.12e-6), (5.58e-5, 1.71e-6)),
+             179.99: ((3.12e-5, 1.75e-6), (3.11e-5, 1.08e-6))}
+
+
+def check_fp32(got, want, fp32):
+    for g, w, (mx, rms) in zip(got, want, fp32):
+        assert np.array_equal(np.isnan(g), np.isnan(w))
+        d = np.abs(g - w)[~np.isnan(w)]
+        print(f"    max-abs {d.max(initial=0.0):.3e}, rms {np.sqrt((d ** 2).sum() / max(1, d.size)):.3e}, "
+              f"{np.isnan(w).mean():.3f} NaN", flush=True)
+        assert d.max(initial=0.0) <= 4 * mx
+        assert (d ** 2).sum() <= (4 * rms) ** 2 * d.size
 
 
 @pytest.mark.parametrize("H,W", [(1, 1), (1, 33), (2, 16), (3, 17), (4, 15), (9, 31), (8, 48),
@@ -76,12 +98,14 @@ def test_large_grids(cuda, H, W):
 def test_hidden_scale(cuda, scale):
     def change(maps):
         maps[2] *= np.float32(scale)
-    check(*run(13, 24, 60.0, 31, change), grow=max(1.0, scale))
+    check_fp32(*run(13, 24, 60.0, 31, change), FP32_SCALE)
 
 
-def test_wide_field_of_view(cuda):
-    """u reaches 572: the maps go through the fp32 products."""
-    check(*run(13, 24, 179.8, 37), grow=572.0)
+@pytest.mark.parametrize("fov", [179.8, 179.99])
+def test_wide_field_of_view(cuda, fov):
+    """u reaches 572, which the maps' scales take, and 11,459, past the largest
+    scale beside these weights."""
+    check_fp32(*run(13, 24, fov, 37), FP32_WIDE[fov])
 
 
 @pytest.mark.parametrize("which,value", [(2, np.nan), (2, np.inf), (1, -np.inf)])
@@ -96,23 +120,6 @@ def test_non_finite_medium(cuda):
     def change(maps):
         maps[2][7, 10, 3] = np.inf
     check(*run(62, 97, 60.0, 43, change))
-
-
-# (max-abs, rms) of result and coarse that convolutions in plain fp32 matrix
-# products (csrc/conv.hip) show against the restatement, at most, over the
-# inputs of the tests that use them: a pixel with a small xy pair amplifies its
-# heads' rounding, so the rms says more.  The bars are four times these.
-FP32_INFINITE = ((1.44e-5, 4.7e-7), (7.44e-4, 3.4e-6))
-
-
-def check_fp32(got, want, fp32):
-    for g, w, (mx, rms) in zip(got, want, fp32):
-        assert np.array_equal(np.isnan(g), np.isnan(w))
-        d = np.abs(g - w)[~np.isnan(w)]
-        print(f"    max-abs {d.max(initial=0.0):.3e}, rms {np.sqrt((d ** 2).sum() / max(1, d.size)):.3e}, "
-              f"{np.isnan(w).mean():.3f} NaN", flush=True)
-        assert d.max(initial=0.0) <= 4 * mx
-        assert (d ** 2).sum() <= (4 * rms) ** 2 * d.size
 
 
 INFINITE = [
@@ -134,6 +141,66 @@ def test_infinite_weight(cuda, H, W, name, at):
     def change(w):
         w[name][at] = np.inf
     check_fp32(*run(H, W, 60.0, 41, change_weights=change), FP32_INFINITE)
+
+
+# One large value in a feature (1) or hidden (2) map: grids of all sets of
+# tiles, magnitudes on both sides of the split form's range, and the hidden
+# map's first row, whose windows reach over the border.
+OUTLIERS = [(16, 80, which, at, v) for which in (1, 2) for at in ((7, 10, 0),)
+            for v in (3e3, 3e4, 1e7, -1e10, 1e18, 1e30)]
+OUTLIERS += [(H, W, which, (33, 0, 40), v) for H, W in ((60, 64), (60, 80), (62, 97), (161, 256))
+             for which, v in ((1, 1e10), (2, -1e7))]
+
+
+@pytest.mark.parametrize("H,W,which,at,value", OUTLIERS)
+def test_outlier(cuda, H, W, which, at, value):
+    """A finite value far above the rest of its map costs no other pixel its
+    precision."""
+    def change(maps):
+        maps[which][at] = value
+    check_fp32(*run(H, W, 60.0, 41, change), FP32_SPREAD)
+
+
+# Spreads that one scale a map cannot hold: a channel far above the others with
+# weights as far below theirs, a region far below the rest that large weights
+# bring back, a map far from unit scale throughout.
+def big_channel(maps, w):
+    maps[1][9] *= np.float32(1e9)
+    for g in "zrq":
+        w[f"gru.conv{g}.weight"][:, 64 + 9] *= np.float32(1e-9)
+
+
+def dim_region(maps, w):
+    one = maps[1][5].copy()
+    maps[1][:, :, :30] = 0
+    maps[1][:, :, 30:] *= np.float32(1e-9)
+    maps[1][5, :, :30], maps[1][5, :, 30:] = one[:, :30], 0
+    for g in "zrq":
+        w[f"gru.conv{g}.weight"][:, np.r_[64:69, 70:128]] *= np.float32(1e9)
+
+
+def large_features(maps, w):
+    maps[1] *= np.float32(1e9)
+    for g in "zrq":
+        w[f"gru.conv{g}.weight"][:, 64:128] *= np.float32(1e-9)
+
+
+def large_head_weights(maps, w):
+    for g in "zr":
+        w[f"gru.conv{g}.weight"] *= np.float32(0.01)
+    w["gru.convq.weight"] *= np.float32(1e-6)
+    w["gru.convq.bias"] *= np.float32(1e-6)
+    maps[2] *= np.float32(1e-6)
+    for h in ("prob", "xy", "angle", "up_prob"):
+        w[f"{h}_head.0.weight"][:, :64] *= np.float32(1e6)
+
+
+@pytest.mark.parametrize("spread", [big_channel, dim_region, large_features, large_head_weights],
+                         ids=lambda f: f.__name__)
+@pytest.mark.parametrize("H,W", [(20, 70), (62, 97), (161, 256)])
+def test_spread(cuda, H, W, spread):
+    """What weights and maps of opposite scales give."""
+    check_fp32(*run(H, W, 60.0, 41, change_both=spread), FP32_SPREAD)
 
 
 @pytest.mark.parametrize("H,W", [(13, 19), (62, 97), (161, 249)])
