@@ -86,9 +86,18 @@ constexpr uint32_t kInfBits = 0x7f800000u;
 // a gate's argument of unit scale.  Values up to 2^13 times unit scale fit
 // beside weights of the usual +-1/sqrt(fan_in).
 constexpr int kBudget = 8;
-__device__ __forceinline__ uint32_t limit_bits(uint32_t wmax) {
-    const int e = 2 * 127 + kBudget - (int)(wmax >> 23);  // (at least 8: wmax is finite)
+// The bits of the largest power of two that times wmax (finite) stays below
+// 2^(budget + 1), at most 2^64.
+__device__ __forceinline__ uint32_t limit_bits(uint32_t wmax, int budget) {
+    const int e = 2 * 127 + budget - (int)(wmax >> 23);  // (at least `budget`)
     return (uint32_t)(e < 191 ? e : 191) << 23;
+}
+// The same for a pixel's activations, which its largest one scales, and the 64
+// inputs of a 1x1 layer: the sums are off by 2^-40 2^11 sqrt(64) / 3 = 2^-27.6.
+// From the limit on, and at an infinity or a NaN, a row takes fp32 products.
+constexpr int kHeadBudget = 10;
+__device__ __forceinline__ uint32_t head_limit(uint32_t wmax) {
+    return wmax < kInfBits ? limit_bits(wmax, kHeadBudget) : 0u;
 }
 
 // The power of two that brings a magnitude of these bits into [2^14, 2^15),
@@ -558,8 +567,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         // A 1x1 layer's reduction step of 32 channels takes M-blocks 2q and
         // 2q + 1: lane (g, col) holds their channels 16 m + 4 g + r, which is
         // its B operand, the weights being packed in that channel order.  Each
-        // pixel's channels are scaled to their largest and split; a row with an
-        // infinity or a NaN (or weights with one) takes fp32 products.  (The
+        // pixel's channels are scaled to their largest and split (head_limit).  (The
         // waves sharing the layers through LDS, six barriers a workgroup, took
         // 99 us for the three heads at 256 x 256 against 61; two waves a SIMD
         // matter more than what a third shape would save: 85 us where the
@@ -573,8 +581,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         const int nout = c.nout[hd], nob = (nout + 15) / 16;
         const uint32_t head4 = split1x1_head_words(nout);
         const __amdgpu_buffer_rsrc_t r4 = rsrc_of(w4 + head4, (uint32_t)nob * 2 * 2048u);
-        const bool ok2 = reinterpret_cast<const uint32_t*>(w2)[64] < kInfBits;
-        const bool ok4 = reinterpret_cast<const uint32_t*>(w4)[16 * nob] < kInfBits;
+        const uint32_t limit2 = head_limit(reinterpret_cast<const uint32_t*>(w2)[64]);
+        const uint32_t limit4 = head_limit(reinterpret_cast<const uint32_t*>(w4)[16 * nob]);
         auto exact16 = [&](const float* w32, int ob, const v4f (&v)[4]) {
             v4f o = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -604,8 +612,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                 split_to(s, b[q][0], b[q][1]);
             }
         };
-        // t of the wave's rows as operands (or, where one is infinite or NaN,
-        // as fp32 values), its exponents, and the rows that are operands
+        // t of the wave's rows as operands (or, from limit4 on, as fp32 values), its
+        // exponents, and the rows that are operands
         v4u tb[NC][4];
         int ex[NC];
         uint32_t split_rows = 0;
@@ -626,7 +634,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                     }
                 }
                 const uint32_t am = px_max(act);
-                if (ok2 && __all(am < kInfBits)) {
+                if (__all(am < limit2)) {
                     const int n = scale_exp(am);
                     h8 b[2][2];
                     operands(act, pow2(n), b);
@@ -659,7 +667,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
                 }
                 const uint32_t tm = px_max(t);
                 ex[j] = 0;
-                if (ok4 && __all(tm < kInfBits)) {
+                if (__all(tm < limit4)) {
                     const int n = scale_exp(tm);
                     h8 b[2][2];
                     operands(t, pow2(n), b);
@@ -1152,7 +1160,7 @@ __global__ __launch_bounds__(256) void split_kernel(PrologueArgs a, int blocks, 
     for (int k = 0; k < 2; ++k) {
         mx[k] = umax(umax(red[k][0], red[k][1]), umax(red[k][2], red[k][3]));
         const uint32_t all = umax(k == 0 ? umax(mx[k], absbits(1.0f)) : mx[k], absbits(uvmax));
-        const uint32_t limit = limit_bits(wmax[k]) - 1;
+        const uint32_t limit = limit_bits(wmax[k], kBudget) - 1;
         n[k] = scale_exp(all < limit ? all : limit);
         wide[k] = all > limit;
     }

@@ -59,6 +59,7 @@ def check(got, want, grow=1.0):
 # heads' rounding, so the rms says more.  The bars are four times these.
 FP32_INFINITE = ((1.44e-5, 4.7e-7), (7.44e-4, 3.4e-6))
 FP32_SPREAD = ((2.24e-5, 4.9e-7), (4.46e-4, 1.03e-6))
+FP32_HEAD = ((8.46e-6, 3.7e-7), (5.59e-5, 7.4e-7))
 FP32_SCALE = ((3.72e-6, 4.7e-7), (1.83e-5, 1.0e-6))
 FP32_WIDE = {179.8: ((1.44e-5, 1.12e-6), (5.58e-5, 1.71e-6)),
              179.99: ((3.12e-5, 1.75e-6), (3.11e-5, 1.08e-6))}
@@ -201,6 +202,33 @@ def large_head_weights(maps, w):
 def test_spread(cuda, H, W, spread):
     """What weights and maps of opposite scales give."""
     check_fp32(*run(H, W, 60.0, 41, change_both=spread), FP32_SPREAD)
+
+
+# One activation of a head far above the others, which the next layer's zero (or
+# as small) weights leave out, and one weight far above the others of its row, on
+# an activation as small.
+def first_activation(w, h):
+    w[h + ".0.bias"][3] = 1e10
+    w[h + ".2.weight"][:, 3] = 0
+
+
+def second_activation(w, h):
+    w[h + ".2.bias"][9] = 1e9
+    w[h + ".4.weight"][:, 9] *= np.float32(1e-9)
+
+
+def one_weight(w, h):
+    w[h + ".0.weight"][5] *= np.float32(1e-10)
+    w[h + ".0.bias"][5] *= np.float32(1e-10)
+    w[h + ".2.weight"][:, 5] *= np.float32(1e10)
+
+
+@pytest.mark.parametrize("spread", [first_activation, second_activation, one_weight],
+                         ids=lambda f: f.__name__)
+@pytest.mark.parametrize("head", ["prob_head", "xy_head", "angle_head", "up_prob_head"])
+@pytest.mark.parametrize("H,W", [(20, 70), (62, 97)])
+def test_head_spread(cuda, H, W, head, spread):
+    check_fp32(*run(H, W, 60.0, 41, change_weights=lambda w: spread(w, head)), FP32_HEAD)
 
 
 @pytest.mark.parametrize("H,W", [(13, 19), (62, 97), (161, 249)])
