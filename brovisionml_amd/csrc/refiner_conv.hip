@@ -359,7 +359,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
     __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads
     __syncthreads();
 
-    if (!exact) {
+    if (__builtin_expect(!exact, 1)) {
         const char* const hb = lds + (g * HSP + wn * NB * HC + col) * 16;
         h8 bw[2][NB][2];
         auto b_load = [&](int st, int slot) {
@@ -432,7 +432,7 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
             }
         }
         // a window holds a value beyond the scale, an infinity or a NaN
-        if (wide) {
+        if (__builtin_expect(wide, 0)) {
             bool bad = false;
 #pragma unroll
             for (int m = 0; m < MB; ++m)
@@ -445,6 +445,86 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         }
     }
 
+    if constexpr (KS > 1) {
+        __syncthreads();  // every wave is done with the halo
+        // (the waves that split the reduction decide together)
+        if (__builtin_expect(wide, 0)) exact = __builtin_amdgcn_readfirstlane(*redo) != 0;
+    }
+    if (__builtin_expect(exact, 0)) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        // fp32 products of the fp32 map and the unsplit weights: one 16x16x4
+        // step per tap and 4 channels.  A row of taps is in flight through the
+        // products of the one before it (each step waiting for its own loads took
+        // a forward with one infinite hidden value at 256 x 256 to 3863 us, so
+        // 2573).  (Buffer loads: 0 beyond the map, by their offset.)
+        constexpr int GROUPS = split_groups(TAIL), ROWS = 16 / KS * K;
+        const __amdgpu_buffer_rsrc_t rw = rsrc_of(
+            c.wp + whead + (size_t)a.wblocks * STEPS * 512,
+            (uint32_t)a.wblocks * TAPS * GROUPS * 256u);
+        const __amdgpu_buffer_rsrc_t rx = rsrc_of(c.x32, 256u * a.HW);
+        float af[2][K][MB], bf[2][K][NB];
+        auto row_load = [&](__amdgpu_buffer_rsrc_t rm, uint32_t px_bytes, uint32_t base, bool use,
+                            int cg, int ky, int slot) {
+#pragma unroll
+            for (int kx = 0; kx < K; ++kx) {
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+                    af[slot][kx][m] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   rw, 4 * lane,
+                                   (((mb0 + m) * GROUPS + cg) * TAPS + ky * K + kx) * 256, 0));
+                const int x = tx0 + col + kx - P;
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                    const int y = ty0 + wn * NB + n + ky - P;
+                    const bool in = use && y >= 0 && y < H && x >= 0 && x < W;
+                    const uint32_t at = base + px_bytes * (uint32_t)(y * W + x);
+                    bf[slot][kx][n] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   rm, (int)(in ? at : 0xf0000000u), 0, 0));
+                }
+            }
+        };
+        auto row_products = [&](int slot) {
+#pragma unroll
+            for (int kx = 0; kx < K; ++kx)
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            af[slot][kx][m], bf[slot][kx][n], acc[m][n], 0, 0, 0);
+        };
+        auto load = [&](int i, int slot) {
+            i = i < ROWS ? i : ROWS - 1;
+            const int cg = ks + i / K * KS;
+            // channel 4 cg + g: NCHW in the context's map, c4 in the others'
+            const uint32_t base = EPI == kPlain ? 4u * (4 * cg + g) * a.HW : 16u * cg * a.HW + 4 * g;
+            row_load(rx, EPI == kPlain ? 4 : 16, base, true, cg, i % K, slot);
+        };
+        static_assert(ROWS % 2 == 0, "two rows a round");
+        load(0, 0);
+        for (int i = 0; i < ROWS; i += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                load(i + u + 1, (u + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+                row_products(u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (TAIL) {
+            const __amdgpu_buffer_rsrc_t ru = rsrc_of(c.uv, 8u * a.HW);
+            if (ks == 0)
+                for (int ky = 0; ky < K; ++ky) {
+                    row_load(ru, 4, 4u * g * a.HW, g < 2, 16, ky, 0);
+                    row_products(0);
+                }
+        }
+    }
     // the heads' second layer's weights, in flight through what follows
     constexpr uint32_t kHead64 = split1x1_head_words(64);
     h8 w2v[HEAD ? 4 : 1][2][2];
@@ -456,52 +536,10 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         }
     };
     const int hd = EPI == kUp ? 3 : HEAD ? mg * WM + wm : 0;
-    auto w2_load = [&]() {
-        if constexpr (HEAD) {
-            const __amdgpu_buffer_rsrc_t r2 = rsrc_of(c.w2[hd] + kHead64, 4 * 2 * 2048u);
+    if constexpr (HEAD) {
+        const __amdgpu_buffer_rsrc_t r2 = rsrc_of(c.w2[hd] + kHead64, 4 * 2 * 2048u);
 #pragma unroll
-            for (int mo = 0; mo < 4; ++mo) w_load(r2, mo, w2v[mo]);
-        }
-    };
-    w2_load();
-
-    if constexpr (KS > 1) {
-        __syncthreads();  // every wave is done with the halo
-        exact = *redo != 0;  // (the waves that split the reduction, together)
-    }
-    if (exact) {
-#pragma unroll
-        for (int m = 0; m < MB; ++m)
-#pragma unroll
-            for (int n = 0; n < NB; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        // fp32 products of the fp32 map and the unsplit weights: one 16x16x4
-        // step per tap and 4 channels
-        constexpr int GROUPS = split_groups(TAIL);
-        const float* const w32 = c.wp + whead + (size_t)a.wblocks * STEPS * 512;
-        for (int cg = ks; cg < GROUPS; cg += KS) {
-            const bool tail = cg == 16;
-            for (int tap = 0; tap < TAPS; ++tap) {
-                float af[MB];
-#pragma unroll
-                for (int m = 0; m < MB; ++m)
-                    af[m] = w32[(((size_t)(mb0 + m) * GROUPS + cg) * TAPS + tap) * 64 + lane];
-#pragma unroll
-                for (int n = 0; n < NB; ++n) {
-                    const int y = ty0 + wn * NB + n + tap / K - P, x = tx0 + col + tap % K - P;
-                    const bool in = y >= 0 && y < H && x >= 0 && x < W && !(tail && g >= 2);
-                    const size_t px = in ? (uint32_t)(y * W + x) : 0u;
-                    const float f = TAIL && tail ? c.uv[(g < 2 ? g : 0) * HW + px]
-                                    : EPI == kPlain ? c.x32[((size_t)4 * cg + g) * HW + px]
-                                                    : c.x32[((size_t)cg * HW + px) * 4 + g];
-                    const float bf = in ? f : 0.0f;
-#pragma unroll
-                    for (int m = 0; m < MB; ++m)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[m], bf, acc[m][n], 0,
-                                                                        0, 0);
-                }
-            }
-        }
-        w2_load();  // (so that they need no registers in these loops)
+        for (int mo = 0; mo < 4; ++mo) w_load(r2, mo, w2v[mo]);
     }
 
     // the groups' partial sums meet: group ks finishes columns n = ks, ks + KS, ...
