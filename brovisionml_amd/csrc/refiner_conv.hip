@@ -82,10 +82,11 @@ constexpr uint32_t kInfBits = 0x7f800000u;
 // Where a map's scale ends: its bound, times the largest weight of the layers
 // that read it, is at most 2^(kBudget + 1).  A value below the bound is off by at
 // most 2^-40 of it, so a sum of 1,650 products with weights spread up to the
-// largest by about 2^-40 2^9 sqrt(1650) / 3 = 2^-27 (rms), below the rounding of
-// a gate's argument of unit scale.  Values up to 2^13 times unit scale fit
-// beside weights of the usual +-1/sqrt(fan_in).
-constexpr int kBudget = 8;
+// largest by about 2^-40 2^11 sqrt(1650) / 3 = 2^-25 (rms): the rounding of a
+// gate of unit scale, a tenth of what an fp32 sum of so many terms is off.
+// Features up to 2^16 fit beside weights of the usual +-1/sqrt(fan_in), up to
+// 2^9 beside a weight of 2.
+constexpr int kBudget = 10;
 // The bits of the largest power of two that times wmax (finite) stays below
 // 2^(budget + 1), at most 2^64.
 __device__ __forceinline__ uint32_t limit_bits(uint32_t wmax, int budget) {

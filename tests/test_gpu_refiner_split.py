@@ -62,7 +62,8 @@ FP32_SPREAD = ((2.24e-5, 4.9e-7), (4.46e-4, 1.03e-6))
 FP32_HEAD = ((8.46e-6, 3.7e-7), (5.59e-5, 7.4e-7))
 FP32_SCALE = ((3.72e-6, 4.7e-7), (1.83e-5, 1.0e-6))
 FP32_WIDE = {179.8: ((1.44e-5, 1.12e-6), (5.58e-5, 1.71e-6)),
-             179.99: ((3.12e-5, 1.75e-6), (3.11e-5, 1.08e-6))}
+             179.99: ((3.12e-5, 1.75e-6), (3.11e-5, 1.08e-6)),
+             179.999: ((8.33e-5, 3.32e-6), (3.36e-5, 1.85e-6))}
 
 
 def check_fp32(got, want, fp32):
@@ -102,10 +103,10 @@ def test_hidden_scale(cuda, scale):
     check_fp32(*run(13, 24, 60.0, 31, change), FP32_SCALE)
 
 
-@pytest.mark.parametrize("fov", [179.8, 179.99])
+@pytest.mark.parametrize("fov", [179.8, 179.99, 179.999])
 def test_wide_field_of_view(cuda, fov):
-    """u reaches 572, which the maps' scales take, and 11,459, past the largest
-    scale beside these weights."""
+    """u reaches 572 and 11,459, which the maps' scales take, and 114,592, past the
+    largest scale beside these weights."""
     check_fp32(*run(13, 24, fov, 37), FP32_WIDE[fov])
 
 
@@ -148,7 +149,7 @@ def test_infinite_weight(cuda, H, W, name, at):
 # tiles, magnitudes on both sides of the split form's range, and the hidden
 # map's first row, whose windows reach over the border.
 OUTLIERS = [(16, 80, which, at, v) for which in (1, 2) for at in ((7, 10, 0),)
-            for v in (3e3, 3e4, 1e7, -1e10, 1e18, 1e30)]
+            for v in (3e3, 6e4, 1e5, 1e7, -1e10, 1e18, 1e30)]
 OUTLIERS += [(H, W, which, (33, 0, 40), v) for H, W in ((60, 64), (60, 80), (62, 97), (161, 256))
              for which, v in ((1, 1e10), (2, -1e7))]
 
