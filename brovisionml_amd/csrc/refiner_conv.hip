@@ -1279,6 +1279,8 @@ hipError_t prologue(const PrologueArgs& a, hipStream_t stream) {
 //            128x160(320) 160x200(520) 200x200(650) 256x256(1024)
 //   Medium     472          727          800          1172
 //   Large      486          759          805          1044
+// Where the lines lie is measured: Medium against Large 801 and 818 us at 650
+// tiles, 830 and 823 at 672, 853 and 848 at 704.
 // Gates and heads in one launch (they depend on the same hidden state only):
 // 19.1 against 12.0 + 11.0 us at 60x80 (Small), 130 against 76 + 64 us at 256x256.
 //                               K  TAIL  MB NB WM WN KS AD EPI
@@ -1294,10 +1296,14 @@ struct Small {
     using Update = Shape<5, false, 2, 4, 1, 1, 4, 4, kUpdate>;
     using Heads = Shape<3, true, 4, 4, 1, 1, 4, 2, kHeads>;
 };
-// Small's gates and heads are 7 workgroups a tile, and the chip holds 512 of
-// them: past 73 tiles gates of twice the channels (5 a tile) avoid a second,
-// nearly empty round (197 against 208 us at 60x80, 75 tiles; 187 against 180 at
-// 50x72, 65).
+// Small's gates and heads are 7 workgroups a tile, and the chip's 256 CUs hold
+// 512 of them: past 73 tiles (512 / 7) gates of twice the channels, 5 a tile, avoid
+// a second, nearly empty round (197 against 208 us at 60x80, 75 tiles; 187
+// against 180 at 50x72, 65).  Its own second round begins past 102 tiles (512 / 5),
+// and the line to Medium, at 110, is a measured one: from 103 tiles to there two
+// cards ran Medium faster by up to 5%, a third SmallFull by up to 3% (60x112, 105
+// tiles: 241 us SmallFull, 230 Medium; 44x160, 110: 243, 241; the third: 229, 228;
+// 230, 236).
 struct SmallFull : Small {
     using Gates = Shape<5, false, 4, 4, 1, 1, 4, 2, kGates>;
 };
@@ -1329,13 +1335,14 @@ hipError_t by_size(const ConvArgs& c, F f) {
 }
 
 // The up-mask head's tiles: one workgroup a CU at a time (its registers), so the
-// fewest rows a workgroup that still fit the chip's 256 in one round; above that
-// the largest tile.  The whole forward against two rows throughout: 130 against
-// 133 us at 13x19, 247 against 253 at 80x100, 334 against 340 at 90x160, 447
-// against 453 at 128x160; four rows at 60x80 take 196 against two's 190.
+// fewest rows a workgroup that still fit the chip's 256 CUs in one round (one row:
+// 4 workgroups a tile); above that the largest tile.  The whole forward against two
+// rows throughout: 130 against 133 us at 13x19, 170 against 173 at 36x96 (54
+// tiles), 247 against 253 at 80x100, 334 against 340 at 90x160, 447 against 453 at
+// 128x160; four rows at 60x80 take 196 against two's 190.
 hipError_t up(const ConvArgs& c, hipStream_t stream) {
     const long long tiles = tiles_of(c);
-    if (tiles <= 48) return launch<Shape<3, true, 4, 1, 1, 1, 4, 2, kUp>>(c, stream);
+    if (tiles <= 64) return launch<Shape<3, true, 4, 1, 1, 1, 4, 2, kUp>>(c, stream);
     if (tiles <= 128) return launch<Shape<3, true, 4, 2, 1, 1, 4, 2, kUp>>(c, stream);
     if (tiles <= 256) return launch<Shape<3, true, 4, 4, 1, 1, 4, 2, kUp>>(c, stream);
     return launch<Shape<3, true, 4, 4, 1, 2, 2, 2, kUp>>(c, stream);

@@ -57,6 +57,10 @@ def check(got, want, grow=1.0):
 # products (csrc/conv.hip) show against the restatement, at most, over the
 # inputs of the tests that use them: a pixel with a small xy pair amplifies its
 # heads' rounding, so the rms says more.  The bars are four times these.
+FP32_LINES = {(32, 128): ((1.51e-6, 1.10e-7), (6.46e-5, 4.4e-7)),
+              (52, 80): ((3.10e-6, 2.03e-7), (2.01e-5, 3.8e-7)),
+              (68, 96): ((2.38e-6, 2.19e-7), (5.70e-5, 5.2e-7)),
+              (52, 128): ((1.75e-5, 1.12e-6), (1.02e-4, 1.74e-6))}
 FP32_INFINITE = ((1.44e-5, 4.7e-7), (7.44e-4, 3.4e-6))
 FP32_SPREAD = ((2.24e-5, 4.9e-7), (4.46e-4, 1.03e-6))
 FP32_HEAD = ((8.46e-6, 3.7e-7), (5.59e-5, 7.4e-7))
@@ -83,6 +87,13 @@ def check_fp32(got, want, fp32):
                                  (62, 128), (63, 129)])
 def test_grids(cuda, H, W):
     check(*run(H, W, 60.0, H + W))
+
+
+@pytest.mark.parametrize("H,W", [(32, 128), (52, 80), (68, 96), (52, 128)])
+def test_grids_at_lines(cuda, H, W):
+    """64 and 65 tiles of 16 x 4, and 102 and 104.  (52 x 128's maps are the
+    ill-conditioned ones.)"""
+    check_fp32(*run(H, W, 60.0, H + W), FP32_LINES[(H, W)])
 
 
 @pytest.mark.parametrize("H,W", [(64, 256), (65, 257), (160, 256), (161, 249)])
