@@ -55,6 +55,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix peak
+F16_MFMA_PEAK_TFLOPS = 2516.6  # MI355X dense f16 matrix peak
 HBM_PEAK_GBPS = 8000.0
 FLUSH_BYTES = 512 << 20
 # Back-to-back work before each timed region, to bring the clocks up (Timer.ramp).
@@ -953,16 +954,24 @@ def bench_upsample(args, dev) -> dict:
 # refiner forward
 # ---------------------------------------------------------------------------
 
-def refiner_kernel_rooflines(dev, H: int, W: int, reps: int):
-    """The refiner's 5x5 ConvGRU convolutions (the implicit-GEMM kernels of
-    brovisionml_amd/csrc/conv.hip) as its forward runs them, each timed alone
-    on the refiner's map size with HIP events on their stream, against the
-    fp32 matrix peak: every iteration convz + convr and convq over the hidden
+def refiner_flops(H: int, W: int) -> int:
+    """The products of one refiner forward, each multiply-add two: the ConvGRU's
+    parts over the 66 constant channels once, those over the hidden state and
+    the three heads every iteration, the up-mask head once."""
+    gru_h, gru_x = 2 * 3 * 64 * 64 * 25, 2 * 3 * 64 * 66 * 25
+    head = 2 * 64 * (66 * 9 + 64)
+    return H * W * (gru_x + 5 * (gru_h + 3 * head + 2 * 64 * 100) + head + 2 * 64 * 576)
+
+
+def abi_convolution_rooflines(dev, H: int, W: int, reps: int):
+    """The C ABI's fp32 5x5 ConvGRU convolutions (brovisionml_amd/csrc/conv.hip;
+    the native refiner runs refiner_conv.hip's kernels instead), each timed
+    alone on the refiner's map size with HIP events on their stream, against the
+    fp32 matrix peak: convz + convr and convq over the hidden
     state's 64 channels (cin 64; the gates and the update in their
-    epilogues, with the part over the other 66 channels added), and once per
-    forward those parts over [feature | uv] (cin 66, plain convolutions).
-    Algorithmic flops per launch = 2 * cout * cin * 25 * H * W.  Returns (the
-    per-iteration convz + convr kernel's roofline, every kernel's figures)."""
+    epilogues, with the part over the other 66 channels added), and
+    those parts over [feature | uv] (cin 66, plain convolutions).
+    Algorithmic flops per launch = 2 * cout * cin * 25 * H * W."""
     import torch
     from brovisionml_amd import _lib
     lib = _lib.load()
@@ -1010,11 +1019,11 @@ def refiner_kernel_rooflines(dev, H: int, W: int, reps: int):
         call()
     out = {}
     for name, (flops, call) in calls.items():
-        # each kernel back to back for RAMP_SECONDS first: the clocks drop
+        # each kernel back to back for the ramp first: the clocks drop
         # while the host packs the weights, and the first kernel timed would
         # otherwise run on the ramp (convz + convr 248 against 233 us)
         t0 = time.perf_counter()
-        while time.perf_counter() - t0 < RAMP_SECONDS:
+        while time.perf_counter() - t0 < Timer.ramp_seconds:
             for _ in range(10):
                 call()
             torch.cuda.synchronize()
@@ -1028,12 +1037,7 @@ def refiner_kernel_rooflines(dev, H: int, W: int, reps: int):
         tf = flops / t / 1e12
         out[name] = {"us": round(t * 1e6, 1), "tflops": round(tf, 1),
                      "frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4), "flops": flops}
-    first = next(iter(out))
-    r = out[first]
-    roof = {"bound": "mfma", "achieved": r["tflops"], "peak": FP32_MFMA_PEAK_TFLOPS,
-            "unit": "TFLOP/s", "frac": r["frac"], "traffic": None, "kernel": first,
-            "flops_per_launch": r["flops"], "launch_us_mean": r["us"]}
-    return roof, out
+    return out
 
 
 def bench_refiner(args, dev) -> dict:
@@ -1041,8 +1045,10 @@ def bench_refiner(args, dev) -> dict:
     synthetic weights and decoder outputs, one forward per step, `steps`
     forwards captured in one graph: the native refiner
     (libbvml_dsine_refine.so: the loop in C++, every convolution on the
-    package's fp32 matrix-core kernels, the propagate with fused activations
-    and the upsample + normalise; the line's value) and the Python driver
+    package's split-half f16 matrix-core kernels, the propagate with fused
+    activations, the up-mask head with the upsample + normalise; the line's
+    value and its roofline, three f16 products a product of the whole forward
+    against the f16 matrix peak) and the Python driver
     (brovisionml_amd/refiner.py: torch's im2col + GEMM convolutions, the
     package's other kernels, with the up-mask head and upsample in every
     iteration) beside it.  The CPU leg is
@@ -1099,12 +1105,22 @@ def bench_refiner(args, dev) -> dict:
                      {"workload": f"dsine-refiner-{H}x{W}", "H": H, "W": W, "iterations": 5,
                       "weights": "synthetic (uniform +-1/sqrt(fan_in))",
                       "driver": driver,
-                      "convolutions": "5x5 and 3x3: implicit-GEMM split-half f16 MFMA kernels, fp32 precision; the "
-                                      "ConvGRU's parts over [feature, uv] once per forward"})
+                      "convolutions": "5x5 and 3x3: implicit-GEMM split-half f16 MFMA kernels, fp32 "
+                                      "precision; the ConvGRU's parts over [feature, uv] once "
+                                      "per forward"})
     if t_py is not None:
         line["python_driver"] = {"ms_per_step": round(t_py * 1e3 / args.steps, 4),
                                  "value": round(opx / t_py / 1e6, 2)}
-    line["roofline"], line["kernels"] = refiner_kernel_rooflines(dev, H, W, args.steps)
+    if args.driver != "python":
+        flops = refiner_flops(H, W)
+        tf = 3 * flops * args.steps / t / 1e12
+        line["roofline"] = {"bound": "mfma", "achieved": round(tf, 1),
+                            "peak": F16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
+                            "frac": round(tf / F16_MFMA_PEAK_TFLOPS, 4), "traffic": None,
+                            "kernel": "the whole forward, three f16 products a product",
+                            "flops_per_launch": 3 * flops,
+                            "launch_us_mean": round(t * 1e6 / args.steps, 1)}
+    line["c_abi_fp32_convolutions"] = abi_convolution_rooflines(dev, H, W, args.steps)
     line["gpu"] = torch.cuda.get_device_name(dev)
     if not args.no_cpu:
         import oracle.refiner as oref

@@ -235,16 +235,6 @@ def convex_upsample_f32(x: int, mask: int, B: int, C: int, H: int, W: int, scale
                                                  eps, out, flags, stream)
 
 
-def convex_upsample_bias_f32(x: int, mask: int, mask_bias: int, B: int, C: int, H: int, W: int,
-                             scale: int, normalize: bool, eps: float, out: int,
-                             flags: int = DEFAULT, stream: int = 0) -> int:
-    """Raw call with a per-channel mask bias (0 for none); pointers are
-    integer device addresses. Returns the status."""
-    return load().bvml_dsine_convex_upsample_bias_f32(x, mask, mask_bias, B, C, H, W, scale,
-                                                      int(bool(normalize)), eps, out, flags,
-                                                      stream)
-
-
 def angmf_recompute_ratio(k: int, flags: int = DEFAULT) -> float:
     """The fast path's cancellation threshold at window size k: pixels with
     |acc|^2 below this times sum (prob/|p|)^2 are recomputed in double (0
