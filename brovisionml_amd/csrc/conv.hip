@@ -1,6 +1,7 @@
 // The refiner's k x k convolutions (k = 3, 5; stride 1, zero "same" padding)
-// as implicit GEMMs on the fp32 matrix cores (the C ABI's bvml_dsine_conv_*):
-// rows = output channels, columns = pixels, the reduction over (input
+// as implicit GEMMs on the fp32 matrix cores (the C ABI's bvml_dsine_conv_*,
+// for callers with a loop of their own; the native refiner's are in
+// refiner_conv.hip): rows = output channels, columns = pixels, the reduction over (input
 // channel, tap).  No im2col buffer: a workgroup of 4 waves owns a 16 x 16
 // pixel tile and 64 or 128 output channels (each wave 64 channels x 4 or 8
 // tile rows: 16 or 32 accumulator blocks, so each weight load feeds 4 or 8

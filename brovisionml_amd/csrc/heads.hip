@@ -1,6 +1,7 @@
 // The refiner's prediction heads after their first (3x3) layer, fused into one
 // per-pixel pass on the fp32 matrix cores (the C ABI's
-// bvml_dsine_heads_mlp_f32).  Each head of src/dsine_refine.cpp:119-127 is
+// bvml_dsine_heads_mlp_f32; the native refiner's heads are in
+// refiner_conv.hip).  Each head of src/dsine_refine.cpp:119-127 is
 // conv3x3 -> ReLU -> conv1x1 -> ReLU -> conv1x1; the 3x3 layer runs as a
 // convolution without its bias, and for every pixel p and head h this pass
 // computes

@@ -73,8 +73,8 @@ const std::vector<std::vector<float>>& host_weights(const bvml_dsine_refiner* r)
 // ConvGRU convolutions' parts over [feature | uv] (constant through the
 // iterations: convz + convr's 128 channels in their packed order, then
 // convq's 64), the uv map and the two tails, the heads' outputs, the two
-// propagate buffers, the ray map, the full-resolution result before the crop,
-// the scales.
+// propagate buffers, the ray map, the scales.  (fs is r*h in fp32 for an
+// update that may need it, once the context has read the features.)
 struct Maps {
     float *hf, *hs, *rs, *fs, *z, *cf, *uv, *th, *tf, *head[kHeads - 1], *pred[2], *ray, *info;
 };

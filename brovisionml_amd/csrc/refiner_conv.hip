@@ -608,7 +608,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
         // its B operand, the weights being packed in that channel order.  Each
         // pixel's channels are scaled to their largest and split (head_limit).  (The
         // waves sharing the layers through LDS, six barriers a workgroup, took
-        // 99 us for the three heads at 256 x 256 against 61; two waves a SIMD
+        // 99 us for the three heads at 256 x 256 against 61, 56 among a forward's
+        // launches; two waves a SIMD
         // matter more than what a third shape would save: 85 us where the
         // registers allowed one.)
         const int* const pe = reinterpret_cast<const int*>(lds + S::kParamAt) + wm * head_words(EPI);
@@ -814,7 +815,8 @@ __device__ __forceinline__ void conv_group(const KArgs& a, int bx, int nbx, char
             // has all 9 taps of its 4 sub-pixels in registers and no mask is
             // written.  Its weights, 9 blocks of 16 outputs, stay in registers
             // over the rows; the activations come from the waves that have
-            // them through LDS.  256 x 256: 75 us against 97 for the head
+            // them through LDS.  256 x 256: 75 us (73 among a forward's
+            // launches) against 97 for the head
             // writing 151 MB of mask and 42 for the upsample reading them;
             // about half is the upsample's vector arithmetic.
             static_assert(EPI != kUp || S::kWaves == 4, "a quarter of the sub-pixels a wave");
@@ -1282,7 +1284,8 @@ hipError_t prologue(const PrologueArgs& a, hipStream_t stream) {
 // Where the lines lie is measured: Medium against Large 801 and 818 us at 650
 // tiles, 830 and 823 at 672, 853 and 848 at 704.
 // Gates and heads in one launch (they depend on the same hidden state only):
-// 19.1 against 12.0 + 11.0 us at 60x80 (Small), 130 against 76 + 64 us at 256x256.
+// 19.1 against 12.0 + 11.0 us at 60x80 (Small), 130 against 76 + 64 us at 256x256
+// (116 against 70 + 56 among a forward's launches, the clock up).
 //                               K  TAIL  MB NB WM WN KS AD EPI
 struct Tiny {
     using Context = Shape<5, true, 4, 2, 1, 1, 4, 2, kPlain>;

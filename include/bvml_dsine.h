@@ -287,7 +287,10 @@ long long bvml_dsine_heads_packed_size(int out);
  *     the hidden state (each sum still fp32, in another order)
  * Outputs must not overlap x (or, for the fused ones, the other inputs and
  * each other).  No counterpart in the reference (brotensor's conv2d_forward
- * followed by its elementwise ops).
+ * followed by its elementwise ops).  These, and the heads' calls above and
+ * below, are for callers with a loop of their own: the native refiner
+ * (bvml_dsine_refine.h) runs other kernels, about three times as fast on a
+ * 256 x 256 grid.
  */
 long long bvml_dsine_conv_packed_size(int cout, int cin, int k);
 int bvml_dsine_conv_pack_f32(const float* w, int cout, int cin, int k, int interleave,

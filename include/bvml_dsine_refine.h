@@ -4,22 +4,25 @@
  *
  * It replaces brovisionml's Refiner (the reference's
  * include/brovisionml/dsine_refine.h:113-145, src/dsine_refine.cpp:161-294):
- * the same weights, the same loop and the same result, in C++ over this
- * library's kernels (bvml_dsine.h) -- RayReLU, the ConvGRU's 5x5
- * convolutions as fp32 matrix-core implicit GEMMs with the gates and the
- * update fused, the heads after their 3x3 layer in one fused pass, the
- * propagate on the heads' raw logits, the convex upsample with its mask
- * bias -- and the heads' 3x3 layer on the same fp32 matrix-core convolution.
- * Its kernels and their launch shapes depend on the grid size only, so a
- * forward gives the same bits in every process.  The C++ class of
+ * the same weights, the same loop and the same result, in C++ over kernels of
+ * its own -- the ConvGRU's 5x5 and the heads' 3x3 convolutions as implicit
+ * GEMMs on the f16 matrix cores at fp32 precision (every operand two halfs),
+ * the gates, the update and the heads' 1x1 layers in their epilogues, the
+ * up-mask head with the convex upsample, normalise and crop -- and
+ * bvml_dsine.h's propagate on the heads' raw logits.  Its kernels and their
+ * launch shapes depend on the grid size only, so a forward gives the same bits
+ * in every process.  Values far beyond the rest of their map (features and
+ * hidden states of 2^16 and more beside weights of the usual initialisation,
+ * infinities, NaN) are convolved in fp32 on the fp32 matrix cores, tile by tile:
+ * the same precision, a slower forward.  The C++ class of
  * include/brovisionml/dsine_refine.h sits on top of it.
  *
  * Lifecycle: create (no HIP call) -> weights (load_file, or set_tensor per
  * tensor) -> forward, any number of times, at any grid size -> destroy.
  * The first forward binds the refiner to the calling thread's current HIP
  * device; later forwards make that device current and restore the caller's.
- * The first forward after a weight change uploads the weights (a
- * synchronous copy, after the device has finished any forward still
+ * The first forward after a weight change uploads the weights and packs them
+ * on the device (synchronously, after the device has finished any forward still
  * reading the old weights), and the first forward at a grid size allocates
  * its buffers (after the device has finished any forward still using the
  * previous size's): run one forward eagerly before capturing forwards into
@@ -127,8 +130,8 @@ int bvml_dsine_refiner_forward_cpu(bvml_dsine_refiner* r, const float* normal,
  * bvml_dsine_refiner_forward: the same result, bit for bit), and the weights
  * must already be on the device: a bvml_dsine_refiner_forward after the last
  * load_file / set_tensor uploads them (else BVML_DSINE_EWEIGHTS).  The array
- * holds 8,388,608 floats (32 MiB) per GPU, the maps of a grid of up to
- * 5,086 pixels (1,649 planes; a 60 x 80 grid needs 7,915,200 floats); a
+ * holds the maps of a grid of up to 5,086 pixels (627 planes, 13 MB per GPU; a
+ * 60 x 80 grid is 4,800 pixels); a
  * larger grid returns BVML_DSINE_ESIZE.  Every call on one GPU uses that
  * GPU's array, which keeps the last call's contents (nothing in it needs to
  * start at zero), so calls on one GPU run in the order they were made: each
