@@ -121,7 +121,7 @@ def test_wide_field_of_view(cuda, fov):
     check_fp32(*run(13, 24, fov, 37), FP32_WIDE[fov])
 
 
-@pytest.mark.parametrize("which,value", [(2, np.nan), (2, np.inf), (1, -np.inf)])
+@pytest.mark.parametrize("which,value", [(2, np.nan), (2, np.inf), (1, -np.inf), (1, np.nan)])
 def test_non_finite(cuda, which, value):
     def change(maps):
         maps[which][7, 10, 3] = value
@@ -241,6 +241,36 @@ def one_weight(w, h):
 @pytest.mark.parametrize("H,W", [(20, 70), (62, 97)])
 def test_head_spread(cuda, H, W, head, spread):
     check_fp32(*run(H, W, 60.0, 41, change_weights=lambda w: spread(w, head)), FP32_HEAD)
+
+
+def test_captured_forward_takes_each_maps_path(cuda):
+    """A forward captured on ordinary maps and replayed on maps with an outlier,
+    an infinity and ordinary ones again gives each the eager forward's bits."""
+    import torch
+    H, W = 45, 64
+    print(f"[gpu] refiner {H}x{W} captured", flush=True)
+    model = rf.NativeRefiner(rf.random_weights(5))
+    intr = wl.intrins_from_fov(8 * H, 8 * W, 60.0)
+    dec = rf.DecoderOutput(*(torch.from_numpy(a)[None].to("cuda:0") for a in pins.inputs(H, W, 5)))
+    ordinary = (dec.feature.clone(), dec.hidden.clone())
+    out = torch.empty((1, 3, 8 * H, 8 * W), device="cuda:0")
+    model.forward(dec, intr, 8 * H, 8 * W, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        model.forward(dec, intr, 8 * H, 8 * W, out=out)
+    for feature, hidden in ((0.0, 0.0), (0.0, 1e10), (np.inf, 0.0), (0.0, 0.0), (1e7, np.inf)):
+        dec.feature.copy_(ordinary[0])
+        dec.hidden.copy_(ordinary[1])
+        if feature:
+            dec.feature[0, 3, 20, 30] = feature
+        if hidden:
+            dec.hidden[0, 7, 10, 3] = hidden
+        want = model.forward(dec, intr, 8 * H, 8 * W)
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
 
 
 @pytest.mark.parametrize("H,W", [(13, 19), (62, 97), (161, 249)])
